@@ -6,104 +6,114 @@
 // hidden_states [T, H] bf16, W [E, H] bf16, b [E] bf16.  The logits then feed
 // the top-k / replay routing (routing.hip).
 //
-// The product is skinny (E = 32 or 128 columns) and reads every activation
-// row once, so it is HBM-bound on x: a block takes 64 rows (two waves of 32)
-// by all E columns.  Each lane loads its A fragments straight from global
-// memory (64 contiguous bytes of one row per 64-deep k-step, one k-step
-// ahead in registers); the W tile of the k-step ([E][64] bf16, 16-byte chunks
-// XOR-swizzled by row) is staged in LDS once per block and shared by both
-// waves, double-buffered.  k is permuted identically on both operands, so
-// lane (r, h) of v_mfma_f32_32x32x16_bf16 feeds k = 32 h + 8 s + (0..7) at
-// sub-step s: a lane's four A fragments are one contiguous 64-byte run.
+// The product is skinny (E = 32 or 128 columns): a block takes 64 rows by all
+// E columns, its waves one 32 x 32 (E > 128: 32 x 64) tile each, and walks k in
+// 64-deep steps.  With one block per CU (16384 rows) or fewer nothing hides a
+// k-step's load latency, and that latency times H / 64 steps is what a plain
+// double buffer costs whatever the row count (33-53 us, 1 row or 16384, where
+// the x read of 16384 rows takes 15 us).  So the x rows ([64][64] bf16) and
+// the W tile ([E][64]) of a k-step go global -> LDS through a ring of kRtStages
+// stages, all but one of them in flight, one barrier per step; the sums keep
+// their order, so the logits are unchanged.  Measured: 1
+// row, E 128 36 -> 16 us; 23 rows, E 32 33 -> 14; 4096 rows, E 32 41 -> 18; 1021
+// rows, E 128 48 -> 24; 16384 rows, E 128 53 -> 30 (LDS reads bound it now).
+// LDS chunks of 16 bytes are XOR-swizzled by row (the copy writes LDS linearly,
+// so the lanes' source addresses carry the swizzle).  k is permuted
+// identically on both operands: lane (r, h) of v_mfma_f32_32x32x16_bf16 feeds
+// k = 32 h + 8 s + (0..7) at sub-step s.
 #include "af3_common.h"
 
 namespace {
 
-constexpr int kRtRows = 64;  // rows per block (2 waves x 32)
+constexpr int kRtRows = 64;  // rows per block
 constexpr int kRtBK = 64;    // k per step
 
-// LDS element offset of 16-byte chunk c of W-tile row n
-__device__ __forceinline__ int rt_off(int n, int c) { return n * kRtBK + ((c ^ (n & 7)) << 3); }
+// one 16-byte global -> LDS copy per lane (LDS address: wave-uniform base + 16 lane)
+__device__ __forceinline__ void rt_dma16(const void* gptr, uint32_t lds_byte_addr) {
+  asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gptr), "{m0}"(lds_byte_addr) : "memory");
+}
 
-template <int TN>
-__global__ __launch_bounds__(128) void router_kernel(const uint16_t* __restrict__ x, int64_t ldx,
-                                                     const uint16_t* __restrict__ w, int64_t ldw,
-                                                     const uint16_t* __restrict__ bias, int64_t T, int H, int E,
-                                                     uint16_t* __restrict__ out, int64_t ldo) {
-  constexpr int EP = TN * 32;                // columns computed (E rounded up to whole sub-tiles)
-  constexpr int WPT = EP * kRtBK / 8 / 128;  // 16-byte W chunks per thread per k-step
-  __shared__ __attribute__((aligned(16))) uint16_t ws[2][EP * kRtBK];
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+// EP columns computed (E rounded up to 32, 64, 128 or 256), TW 32-column tiles per wave, ST ring stages
+template <int EP, int TW, int ST>
+__global__ __launch_bounds__(EP / TW * 4) void router_kernel(const uint16_t* __restrict__ x, int64_t ldx,
+                                                             const uint16_t* __restrict__ w, int64_t ldw,
+                                                             const uint16_t* __restrict__ bias, int64_t T, int H, int E,
+                                                             uint16_t* __restrict__ out, int64_t ldo) {
+  constexpr int NW = EP / TW / 16;                 // waves: 2 row groups x EP / (32 TW) column groups
+  constexpr int STAGE = (kRtRows + EP) * 128;      // bytes: x rows, then W rows
+  constexpr int CPW = (kRtRows + EP) / 8 / NW;     // 1 KB copies (8 rows) per wave and k-step
+  static_assert((kRtRows + EP) / 8 % NW == 0, "whole copies per wave");
+  static_assert(CPW * (ST - 2) <= 31 && ST * STAGE <= 160 * 1024, "ring");
+  __shared__ __attribute__((aligned(16))) uint8_t lds[ST * STAGE];
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int lr = lane & 31, lh = lane >> 5;
-  const int64_t row = (int64_t)blockIdx.x * kRtRows + wave * 32 + lr;
-  const uint16_t* xr = x + (row < T ? row : T - 1) * ldx + lh * 32;
+  const int rg = wave & 1, cg = wave >> 1;
   const int nk = H / kRtBK;
+  const int64_t row0 = (int64_t)blockIdx.x * kRtRows;
+  const bool rows = row0 + rg * 32 < T;  // else the wave only copies and keeps the barriers
 
-  af3_u32x4 xa[4], wv[WPT];
-  auto load_x = [&](int kk) {
+  // copy j of the wave: rows 8 (wave CPW + j) .. + 7 of the stage, lane l row l / 8, 16-byte slot l % 8
+  const uint16_t* src[CPW];
 #pragma unroll
-    for (int s = 0; s < 4; ++s) xa[s] = *(const af3_u32x4*)(xr + kk * kRtBK + s * 8);
-  };
-  auto load_w = [&](int kk) {
+  for (int j = 0; j < CPW; ++j) {
+    const int r = (wave * CPW + j) * 8 + (lane >> 3);
+    const int ch = (lane & 7) ^ (r & 7);
+    if (r < kRtRows)  // rows past T: any valid row (their results are not stored)
+      src[j] = x + min(row0 + r, T - 1) * ldx + ch * 8;
+    else
+      src[j] = w + (int64_t)min(r - kRtRows, E - 1) * ldw + ch * 8;
+  }
+  const uint32_t lds0 = __builtin_amdgcn_readfirstlane(
+      (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)lds);
+  // k-steps past the end copy the last one again, into a stage no wave reads again
+  auto issue = [&](int kk) {
+    const int ks = min(kk, nk - 1);
+    const uint32_t st = lds0 + (uint32_t)((kk % ST) * STAGE + wave * CPW * 1024);
 #pragma unroll
-    for (int j = 0; j < WPT; ++j) {
-      const int id = j * 128 + threadIdx.x;
-      const int n = min(id >> 3, E - 1);  // rows past E: any valid row (their columns are not stored)
-      wv[j] = *(const af3_u32x4*)(w + (int64_t)n * ldw + kk * kRtBK + (id & 7) * 8);
-    }
-  };
-  auto store_w = [&](int buf) {
-#pragma unroll
-    for (int j = 0; j < WPT; ++j) {
-      const int id = j * 128 + threadIdx.x;
-      *(af3_u32x4*)(ws[buf] + rt_off(id >> 3, id & 7)) = wv[j];
-    }
+    for (int j = 0; j < CPW; ++j) rt_dma16(src[j] + ks * kRtBK, st + (uint32_t)(j * 1024));
   };
 
-  af3_f32x16 acc[TN];
+  af3_f32x16 acc[TW];
 #pragma unroll
-  for (int t = 0; t < TN; ++t)
+  for (int t = 0; t < TW; ++t)
 #pragma unroll
     for (int r = 0; r < 16; ++r) acc[t][r] = 0.f;
 
-  load_w(0);
-  load_x(0);
-  store_w(0);
-  __syncthreads();
-  for (int kk = 0; kk < nk; ++kk) {
-    const int buf = kk & 1;
-    af3_u32x4 xc[4];
 #pragma unroll
-    for (int s = 0; s < 4; ++s) xc[s] = xa[s];
-    if (kk + 1 < nk) {  // next k-step's operands in flight during this one's MFMAs
-      load_w(kk + 1);
-      load_x(kk + 1);
-    }
+  for (int k = 0; k < ST - 1; ++k) issue(k);
+  for (int kk = 0; kk < nk; ++kk) {
+    // this wave's copies of k-step kk have landed (those of the ST - 2 newer
+    // steps may be outstanding); then the barrier: every wave's have, and every
+    // wave has read stage kk - 1, which the next copies overwrite
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(CPW * (ST - 2)) : "memory");
+    issue(kk + ST - 1);
+    if (!rows) continue;
+    const uint8_t* const st = lds + (kk % ST) * STAGE;
+    const uint8_t* const ar = st + (rg * 32 + lr) * 128;
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
-      const af3_bf16x8 a = __builtin_bit_cast(af3_bf16x8, xc[s]);
+      const int ch = ((lh * 4 + s) ^ (lr & 7)) << 4;
+      const af3_bf16x8 a = *(const af3_bf16x8*)(ar + ch);
 #pragma unroll
-      for (int t = 0; t < TN; ++t) {
-        const af3_bf16x8 b = *(const af3_bf16x8*)(ws[buf] + rt_off(t * 32 + lr, lh * 4 + s));
+      for (int t = 0; t < TW; ++t) {
+        const af3_bf16x8 b = *(const af3_bf16x8*)(st + (kRtRows + (cg * TW + t) * 32 + lr) * 128 + ch);
         acc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc[t], 0, 0, 0);
       }
     }
-    if (kk + 1 < nk) {
-      store_w(buf ^ 1);  // the other buffer was last read in k-step kk - 1 (before the barrier below it)
-      __syncthreads();
-    }
   }
-  // epilogue: lane (c, h) of sub-tile t holds rows 8 j + 4 h + q, column t * 32 + c
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the repeated last copies, before the LDS is given back
+  // epilogue: lane (c, h) of sub-tile t holds rows 8 j + 4 h + q, column 32 (cg TW + t) + c
 #pragma unroll
-  for (int t = 0; t < TN; ++t) {
-    const int col = t * 32 + lr;
+  for (int t = 0; t < TW; ++t) {
+    const int col = (cg * TW + t) * 32 + lr;
     if (col >= E) continue;
     const float b = bias ? af3_bf16_to_f32(bias[col]) : 0.f;
 #pragma unroll
     for (int j = 0; j < 4; ++j)
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const int64_t r = (int64_t)blockIdx.x * kRtRows + wave * 32 + 8 * j + 4 * lh + q;
+        const int64_t r = row0 + rg * 32 + 8 * j + 4 * lh + q;
         if (r < T) out[r * ldo + col] = (uint16_t)af3_f32_to_bf16(acc[t][4 * j + q] + b);
       }
   }
@@ -123,14 +133,18 @@ extern "C" int af3_router_logits(const uint16_t* x, int64_t ldx, const uint16_t*
               "router_logits: x and W rows must be 16-byte aligned");
   if (n_tokens == 0) return 0;
   AF3_REQUIRE(x && w && logits, "router_logits: null pointer");
-  const dim3 grid((unsigned)af3_cdiv(n_tokens, kRtRows)), block(128);
-  switch ((n_expts + 31) / 32) {
-#define AF3_RT(tn) \
-  case tn:         \
-    hipLaunchKernelGGL(router_kernel<tn>, grid, block, 0, stream, x, ldx, w, ldw, bias, n_tokens, hidden, n_expts, logits, ld_logits); \
-    break;
-    AF3_RT(1) AF3_RT(2) AF3_RT(3) AF3_RT(4) AF3_RT(5) AF3_RT(6) AF3_RT(7) AF3_RT(8)
+  const dim3 grid((unsigned)af3_cdiv(n_tokens, kRtRows));
+#define AF3_RT(ep, tw, st)                                                                                        \
+  hipLaunchKernelGGL((router_kernel<ep, tw, st>), grid, dim3(ep / tw * 4), 0, stream, x, ldx, w, ldw, bias, n_tokens, \
+                     hidden, n_expts, logits, ld_logits)
+  if (n_expts <= 32)
+    AF3_RT(32, 1, 6);   // 12 KB stages, 6 copies per wave and step
+  else if (n_expts <= 64)
+    AF3_RT(64, 1, 8);   // 16 KB, 4
+  else if (n_expts <= 128)
+    AF3_RT(128, 1, 6);  // 24 KB, 3
+  else
+    AF3_RT(256, 2, 4);  // 40 KB, 5
 #undef AF3_RT
-  }
   return af3::check_launch("router_logits");
 }
