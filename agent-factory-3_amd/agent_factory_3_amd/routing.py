@@ -17,6 +17,7 @@ All index work runs in HIP kernels on the caller's stream (no host sync).
 """
 from __future__ import annotations
 
+import ctypes
 from dataclasses import dataclass, field
 
 import torch
@@ -28,6 +29,7 @@ from . import _capi
 BLOCK_MS = (128, 256, 512)
 GEMM_ORDER_BMS = (128,)  # tile sizes whose full-first work order is made with the routing (the
 # default GEMMs and the LoRA row tiles); other sizes get theirs on first use (gemm_order_for)
+PLAN_MAX_E = 1024  # experts of af3_routing_plan (routing and tile metadata in one call)
 
 
 @dataclass
@@ -177,6 +179,39 @@ class _GateScal(torch.autograd.Function):
         return dlogits.to(ctx.dtype), None, None, None, None
 
 
+def _routing_plan(lg: torch.Tensor, K: int, ei: torch.Tensor | None, ld: int):
+    """Routing and its tile metadata in one call (af3_routing_plan): the outputs
+    are slices of one int32 buffer.  Returns (gate_scal, hist, topk_indx,
+    gate_indx, ExptData)."""
+    T, E = lg.shape
+    R = T * K
+    dev = lg.device
+    bms = BLOCK_MS
+    nb = len(bms)
+    tiles = [max_tiles(R, E, bm) for bm in bms]
+    mt = max(tiles)
+    n_ord = max(bms.index(bm) for bm in GEMM_ORDER_BMS) + 1   # orders for the leading sizes
+    sizes = [E, E + 1, R, R] + [E + 1] * nb + [mt] * (nb + n_ord)
+    buf = torch.empty(sum(sizes), dtype=torch.int32, device=dev)
+    gate_scal = torch.empty(R, dtype=torch.bfloat16, device=dev)
+    lib = _capi.load()
+    topk = 1 if ei is None else 0
+    ws_n = int(lib.af3_routing_plan_workspace_bytes(T, E, K, topk))
+    ws = torch.empty(ws_n, dtype=torch.uint8, device=dev) if ws_n else None
+    hist, offs, topk_indx, gate_indx, *rest = buf.split(sizes)
+    _capi.call("af3_routing_plan", lg.data_ptr(), ld, _capi.ptr(ei), topk, T, E, K, gate_scal.data_ptr(),
+               hist.data_ptr(), topk_indx.data_ptr(), gate_indx.data_ptr(), offs.data_ptr(),
+               (ctypes.c_int32 * nb)(*bms), nb, n_ord, mt, rest[0].data_ptr(), rest[nb].data_ptr(),
+               rest[2 * nb].data_ptr(), _capi.ptr(ws), ws_n, _capi.stream_of(dev))
+    ed = ExptData(hist, offs, n_gates=R)
+    for i, bm in enumerate(bms):
+        ed.token_offs_pad[bm] = rest[i]
+        ed.block_pid_map[bm] = rest[nb + i]
+        if i < n_ord:
+            ed.gemm_order[bm] = rest[2 * nb + i][:tiles[i]]
+    return gate_scal, hist, topk_indx, gate_indx, ed
+
+
 def _run_routing(logits: torch.Tensor, n_expts_act: int, expt_indx: torch.Tensor | None):
     out_dtype = logits.dtype
     lg = _bf16_logits(logits)
@@ -184,26 +219,29 @@ def _run_routing(logits: torch.Tensor, n_expts_act: int, expt_indx: torch.Tensor
     K = int(n_expts_act)
     R = T * K
     dev = lg.device
-    gate_scal = torch.empty(R, dtype=torch.bfloat16, device=dev)
-    hist = torch.empty(E, dtype=torch.int32, device=dev)
-    topk_indx = torch.empty(R, dtype=torch.int32, device=dev)
-    gate_indx = torch.empty(R, dtype=torch.int32, device=dev)
-    offs = torch.empty(E + 1, dtype=torch.int32, device=dev)
-    ws_n = _capi.workspace_bytes(T, E, K)
-    ws = torch.empty(ws_n, dtype=torch.uint8, device=dev)
-    stream = _capi.stream_of(dev)
     ld = lg.stride(0) if T > 1 else E
+    ei = None
     if expt_indx is not None:
         ei = expt_indx.to(device=dev, dtype=torch.int32).contiguous()
         if ei.shape != (T, K):
             raise ValueError(f"expt_indx shape {tuple(ei.shape)} != ({T}, {K})")
-        _capi.call("af3_routing_replay", lg.data_ptr(), ld, ei.data_ptr(), T, E, K, gate_scal.data_ptr(),
-                   hist.data_ptr(), topk_indx.data_ptr(), gate_indx.data_ptr(), offs.data_ptr(), ws.data_ptr(),
-                   ws_n, stream)
+    if 0 < E <= PLAN_MAX_E:
+        gate_scal, hist, topk_indx, gate_indx, expt_data = _routing_plan(lg, K, ei, ld)
     else:
-        _capi.call("af3_routing_topk", lg.data_ptr(), ld, T, E, K, gate_scal.data_ptr(), hist.data_ptr(),
-                   topk_indx.data_ptr(), gate_indx.data_ptr(), offs.data_ptr(), ws.data_ptr(), ws_n, stream)
-    expt_data = compute_expt_data(hist, E, R, token_offs_raw=offs)
+        gate_scal = torch.empty(R, dtype=torch.bfloat16, device=dev)
+        hist = torch.empty(E, dtype=torch.int32, device=dev)
+        topk_indx = torch.empty(R, dtype=torch.int32, device=dev)
+        gate_indx = torch.empty(R, dtype=torch.int32, device=dev)
+        offs = torch.empty(E + 1, dtype=torch.int32, device=dev)
+        ws_n = _capi.workspace_bytes(T, E, K)
+        ws = torch.empty(ws_n, dtype=torch.uint8, device=dev)
+        outs = (T, E, K, gate_scal.data_ptr(), hist.data_ptr(), topk_indx.data_ptr(), gate_indx.data_ptr(),
+                offs.data_ptr(), ws.data_ptr(), ws_n, _capi.stream_of(dev))
+        if ei is not None:
+            _capi.call("af3_routing_replay", lg.data_ptr(), ld, ei.data_ptr(), *outs)
+        else:
+            _capi.call("af3_routing_topk", lg.data_ptr(), ld, *outs)
+        expt_data = compute_expt_data(hist, E, R, token_offs_raw=offs)
     if out_dtype != torch.bfloat16 and out_dtype.is_floating_point:
         gate_scal = gate_scal.to(out_dtype)
     if GAMMA_GRAD and torch.is_grad_enabled() and logits.requires_grad:

@@ -16,11 +16,17 @@
 //                    scan of ceil(hist/BM) and block_pid_map[i] = (b<<16)|e for
 //                    the b-th BM-row block of expert e, -1 for unused slots.
 //
-// The sort is a stable counting sort: per 256-entry chunk histograms, a scan
-// over (expert, chunk), then a scatter where each entry's rank among equal ids
-// earlier in its chunk keeps the order of the flat index.  Entries whose
-// expert id is outside [0, E) are dropped (gate_indx = -1), the same shape the
-// reference gives expert-parallel-masked entries.
+// The sort is a stable counting sort: histograms of chunks of the flat index,
+// a scan over (expert, chunk), then a scatter where each entry's rank among
+// equal ids earlier in its chunk keeps the order of the flat index.  Entries
+// whose expert id is outside [0, E) are dropped (gate_indx = -1), the same
+// shape the reference gives expert-parallel-masked entries.
+//
+// Up to 1024 experts the whole chain (ids and weights, sort, tile maps, work
+// orders) is one launch of one block for small batches and three launches
+// otherwise: every step is a few microseconds of latency, so what a call costs
+// is the number of dependent steps, not bytes.  More experts take the older
+// chain of one kernel per step.
 #include <mutex>
 
 #include "af3_common.h"
@@ -214,6 +220,467 @@ __global__ void fill_tail_kernel(const int32_t* __restrict__ offs, int E, int64_
   }
 }
 
+// ---------------------------------------------------------------------------
+// Routing plan for E <= 1024 experts.
+//
+// What bounds it is a chain of short dependent steps, so the steps are merged:
+//   * plan_small_kernel (T K <= 4096 entries): one block does everything;
+//   * larger batches: token_hist_kernel (ids, weights, per-chunk histograms of
+//     64 tokens), plan_scan_kernel (one block: prefix over chunks and experts,
+//     tile maps, work orders), plan_scatter_kernel (stable scatter).
+// A token's 16 lanes hold its E logits (E <= 256) and pick the top K by K
+// max-reductions of (order-preserving logit bits, inverted id) keys, so ties
+// go to the lower id; one thread per token with a sorted insertion took
+// 25-45 us (a serial pass over E with one wave per CU).  The rank of an entry
+// among equal ids of its wave comes from ballots over the id's bits instead of
+// a scan of the chunk.  Measured (4 of E, kernel time per call, from ids and
+// weights to the tile maps and work order): top-k of 23 tokens over 32
+// experts 55 -> 10 us, 4096 tokens 79 -> 26 us, replay of 1021 tokens over 128
+// experts 36 -> 24 us, 16384 tokens 52 -> 33 us.
+// ---------------------------------------------------------------------------
+constexpr int kPlanMaxE = 1024;       // experts (one thread each in the scans)
+constexpr int kPlanMaxTopkE = 256;    // experts of the 16-lane top-k (16 logits per lane)
+constexpr int kPlanSmallR = 4096;     // entries of the one-block plan
+constexpr int kPlanSmallTopkT = 256;  // tokens whose top-k the one-block plan takes along (64 per pass)
+constexpr int kPlanSmallCnt = 16384;  // (64-entry group, expert) counters of the one-block plan (64 KB)
+constexpr int kPlanTokens = 64;       // tokens per chunk of the three-launch plan (one pass of 16-lane groups)
+constexpr int kPlanMaxBm = 8;
+
+// tile maps and work orders to make (n_bm = 0: none); orders for the first n_order sizes
+struct PlanMaps {
+  int n_bm, n_order, max_tiles;
+  int bm[kPlanMaxBm];
+  int32_t *offs_pad, *map, *order;  // [n_bm][E + 1], [n_bm][max_tiles], [n_order][max_tiles]
+};
+
+// bf16 bits -> 16-bit key in float order (-0 as +0; NaN lowest, as a stable descending sort puts it last)
+__device__ __forceinline__ uint32_t plan_key16(uint32_t b) {
+  if ((b & 0x7FFFu) > 0x7F80u) return 0u;
+  if (b == 0x8000u) b = 0u;
+  return (b & 0x8000u) ? (~b & 0xFFFFu) : (b | 0x8000u);
+}
+__device__ __forceinline__ float plan_key_value(uint32_t k16) {
+  const uint32_t b = k16 == 0u ? 0x7FC0u : (k16 & 0x8000u) ? (k16 & 0x7FFFu) : (~k16 & 0xFFFFu);
+  return af3_bf16_to_f32(b);
+}
+
+// The K (id, softmax weight) slots of token t by its 16 lanes (all 64 lanes of
+// the wave must call it; t >= T is idle): lane j < K returns slot j's expert id
+// (-1: dropped) and bf16 weight.  TOPK: slots by ascending id.
+template <bool TOPK>
+__device__ __forceinline__ void plan_token(const uint16_t* __restrict__ logits, int64_t ld,
+                                           const int32_t* __restrict__ idx, int64_t t, int64_t T, int E, int K,
+                                           int32_t& id, uint16_t& w) {
+  const int l = threadIdx.x & 15;
+  const bool on = t < T;
+  float v = -INFINITY;
+  int32_t e = -1;
+  if constexpr (TOPK) {
+    uint32_t key[kPlanMaxTopkE / 16];
+    const uint16_t* row = logits + (on ? t : 0) * ld;
+#pragma unroll
+    for (int i = 0; i < kPlanMaxTopkE / 16; ++i) {
+      const int x = l + 16 * i;
+      key[i] = x < E ? (plan_key16(row[x]) << 16) | (0xFFFFu - (uint32_t)x) : 0u;
+    }
+    uint32_t mine = 0u;
+    for (int j = 0; j < K; ++j) {
+      uint32_t m = 0u;
+#pragma unroll
+      for (int i = 0; i < kPlanMaxTopkE / 16; ++i) m = max(m, key[i]);
+#pragma unroll
+      for (int o = 8; o > 0; o >>= 1) m = max(m, (uint32_t)__shfl_xor((int)m, o, 16));
+#pragma unroll
+      for (int i = 0; i < kPlanMaxTopkE / 16; ++i) key[i] = key[i] == m ? 0u : key[i];
+      if (l == j) mine = m;
+    }
+    v = plan_key_value(mine >> 16);
+    e = (int32_t)(0xFFFFu - (mine & 0xFFFFu));
+  } else if (on && l < K) {
+    e = idx[t * K + l];
+    if (e < 0 || e >= E)
+      e = -1;
+    else
+      v = af3_bf16_to_f32(logits[t * ld + e]);
+  }
+  float mx = TOPK ? __shfl(v, 0, 16) : -INFINITY;
+  if constexpr (!TOPK)
+    for (int j = 0; j < K; ++j) mx = fmaxf(mx, __shfl(v, j, 16));
+  const float x = e >= 0 ? expf(v - mx) : 0.f;
+  float den = 0.f;
+  for (int j = 0; j < K; ++j) den += __shfl(x, j, 16);  // in slot order
+  uint32_t wb = bf16_bits_rne(x / den);
+  if constexpr (TOPK) {  // by ascending id: slot of winner j = winners with a lower id
+    int rank = 0;
+    for (int j = 0; j < K; ++j) rank += __shfl(e, j, 16) < e;
+    int32_t se = -1;
+    uint32_t sw = 0u;
+    for (int j = 0; j < K; ++j) {
+      const int r = __shfl(rank, j, 16);
+      const int32_t ej = __shfl(e, j, 16);
+      const uint32_t wj = (uint32_t)__shfl((int)wb, j, 16);
+      if (r == l) {
+        se = ej;
+        sw = wj;
+      }
+    }
+    e = se;
+    wb = sw;
+  }
+  id = e;
+  w = (uint16_t)wb;
+}
+
+// rank of this lane's id among the equal ids of lower lanes, and how many lanes hold it (e < 0: none)
+__device__ __forceinline__ int plan_wave_rank(int e, int ebits, int& count) {
+  uint64_t m = __ballot(e >= 0);
+  for (int b = 0; b < ebits; ++b) {
+    const uint64_t s = __ballot((e >> b) & 1);
+    m &= ((e >> b) & 1) ? s : ~s;
+  }
+  const int lane = threadIdx.x & 63;
+  count = __popcll(m);
+  return __popcll(m & ((1ull << lane) - 1ull));
+}
+
+// inclusive prefix over a wave
+__device__ __forceinline__ int plan_wave_scan(int v) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const int u = __shfl_up(v, o, 64);
+    if (lane >= o) v += u;
+  }
+  return v;
+}
+
+// padded offsets, tile maps and work orders from the experts' counts (LDS, E
+// ints, published by a barrier).  A block of one CU issues one wave
+// instruction per SIMD and cycle, so work that 128 experts need once is not
+// spread over 16 waves that all run it: wave j makes the tile map of size j,
+// wave n_bm + j the order of size j (the whole block scanning one size after
+// another made plan_scan_kernel 22 us at 4096 tokens of 32 experts, this 14).
+__device__ void plan_maps(const PlanMaps& m, int E, const int32_t* counts) {
+  const int lane = threadIdx.x & 63;
+  const int job = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  if (job >= m.n_bm + m.n_order) return;
+  const bool ord = job >= m.n_bm;
+  const int b = ord ? job - m.n_bm : job;
+  const int bm = m.bm[b];
+  int32_t* const out = (ord ? m.order : m.map) + (int64_t)b * m.max_tiles;
+  int carry = 0;
+  for (int e0 = 0; e0 < E; e0 += 64) {  // (full) tiles in expert order
+    const int e = e0 + lane, h = e < E ? counts[e] : 0;
+    const int n = ord ? h / bm : (h + bm - 1) / bm;
+    const int incl = plan_wave_scan(n), at = carry + incl - n;
+    if (!ord && e < E) m.offs_pad[b * (E + 1) + e] = at;
+    // an expert's first two tiles by its lane, the rest by the wave
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+      if (i < n && at + i < m.max_tiles) out[at + i] = (i << 16) | e;
+    for (uint64_t big = __ballot(n > 2); big; big &= big - 1) {
+      const int l = __ffsll((unsigned long long)big) - 1;
+      const int n_l = __shfl(n, l, 64), at_l = __shfl(at, l, 64);
+      for (int i = 2 + lane; i < n_l; i += 64)
+        if (at_l + i < m.max_tiles) out[at_l + i] = (i << 16) | (e0 + l);
+    }
+    carry += __shfl(incl, 63, 64);
+  }
+  if (!ord && lane == 0) m.offs_pad[b * (E + 1) + E] = carry;
+  if (ord) {  // then the partial tiles by decreasing rows, ties to the lower expert
+    int n_part = 0;
+    for (int e0 = 0; e0 < E; e0 += 64) {
+      const int e = e0 + lane, h = e < E ? counts[e] : 0;
+      const int full = h / bm, mine = h - full * bm;
+      int rank = 0;
+      for (int f0 = 0; f0 < E; f0 += 64) {  // 64 experts' tails at a time, one per lane
+        const int hf = f0 + lane < E ? counts[f0 + lane] : 0;
+        const int tail = hf % bm;
+        if (e0 == 0) n_part += __popcll(__ballot(tail != 0));
+#pragma unroll 8
+        for (int l = 0; l < 64; ++l) {
+          const int x = __builtin_amdgcn_readlane(tail, l);
+          rank += x > mine || (x == mine && f0 + l < e);
+        }
+      }
+      if (mine && carry + rank < m.max_tiles) out[carry + rank] = (full << 16) | e;
+    }
+    carry += n_part;
+  }
+  for (int i = carry + lane; i < m.max_tiles; i += 64) out[i] = -1;
+}
+
+// hist, offs [E + 1] and start (LDS) = the exclusive prefix of the experts' counts (LDS), by one wave; returns the sum
+__device__ __forceinline__ int plan_offsets(int E, int32_t* counts, int32_t* __restrict__ hist,
+                                            int32_t* __restrict__ offs, int32_t* start) {
+  const int lane = threadIdx.x & 63;
+  int carry = 0;
+  for (int e0 = 0; e0 < E; e0 += 64) {
+    const int e = e0 + lane, h = e < E ? counts[e] : 0;
+    const int incl = plan_wave_scan(h);
+    if (e < E) {
+      hist[e] = h;
+      offs[e] = carry + incl - h;
+      start[e] = carry + incl - h;
+    }
+    carry += __shfl(incl, 63, 64);
+  }
+  if (lane == 0) offs[E] = carry;
+  return carry;
+}
+
+// the whole plan in one block. MODE 0: top-k of the logits, 1: given ids, 2: ids / weights already made
+template <int MODE>
+__global__ __launch_bounds__(1024) void plan_small_kernel(const uint16_t* __restrict__ logits, int64_t ld,
+                                                          const int32_t* __restrict__ idx, int T, int E, int K,
+                                                          const int32_t* __restrict__ ids_in,
+                                                          const uint16_t* __restrict__ scal_in, int ebits,
+                                                          uint16_t* __restrict__ gate_scal, int32_t* __restrict__ hist,
+                                                          int32_t* __restrict__ topk_indx,
+                                                          int32_t* __restrict__ gate_indx, int32_t* __restrict__ offs,
+                                                          PlanMaps m) {
+  __shared__ int32_t ids[kPlanSmallR];
+  __shared__ uint16_t sc[kPlanSmallR];
+  __shared__ int32_t cnt[kPlanSmallCnt];  // [64-entry group][E]
+  __shared__ int32_t start[kPlanMaxE];
+  __shared__ int32_t counts[kPlanMaxE];
+  __shared__ int32_t total;
+  const int t = threadIdx.x, R = T * K, ngroup = (R + 63) / 64;
+  if constexpr (MODE == 2) {
+    for (int i = t; i < R; i += 1024) {
+      ids[i] = ids_in[i];
+      sc[i] = scal_in[i];
+    }
+  } else if constexpr (MODE == 0) {
+    for (int t0 = 4 * (t >> 6); t0 < T; t0 += 64) {  // four tokens per wave, idle waves skip
+      const int tok = t0 + ((t & 63) >> 4);
+      int32_t e;
+      uint16_t w;
+      plan_token<true>(logits, ld, idx, tok, T, E, K, e, w);
+      if (tok < T && (t & 15) < K) {
+        ids[tok * K + (t & 15)] = e;
+        sc[tok * K + (t & 15)] = w;
+      }
+    }
+  } else {
+    // replay: every slot's id, then every slot's logit (two loads deep however
+    // many tokens), then one thread per token
+    float* const val = (float*)cnt;
+    int32_t id[kPlanSmallR / 1024];
+#pragma unroll
+    for (int q = 0; q < kPlanSmallR / 1024; ++q) {
+      const int i = q * 1024 + t;
+      id[q] = i < R ? idx[i] : -1;
+    }
+#pragma unroll
+    for (int q = 0; q < kPlanSmallR / 1024; ++q) {
+      const int i = q * 1024 + t;
+      const bool ok = id[q] >= 0 && id[q] < E;
+      const float v = ok ? af3_bf16_to_f32(logits[(int64_t)(i / K) * ld + id[q]]) : -INFINITY;
+      if (i < R) {
+        ids[i] = ok ? id[q] : -1;
+        val[i] = v;
+      }
+    }
+    __syncthreads();
+    for (int tok = t; tok < T; tok += 1024) {
+      float mx = -INFINITY, den = 0.f;
+      for (int j = 0; j < K; ++j) mx = fmaxf(mx, val[tok * K + j]);
+      for (int j = 0; j < K; ++j) {
+        const float x = ids[tok * K + j] >= 0 ? expf(val[tok * K + j] - mx) : 0.f;
+        val[tok * K + j] = x;
+        den += x;
+      }
+      for (int j = 0; j < K; ++j) sc[tok * K + j] = (uint16_t)bf16_bits_rne(val[tok * K + j] / den);
+    }
+    __syncthreads();
+  }
+  for (int i = t; i < ngroup * E; i += 1024) cnt[i] = 0;
+  __syncthreads();
+  int rank[kPlanSmallR / 1024];
+#pragma unroll
+  for (int q = 0; q < kPlanSmallR / 1024; ++q) {
+    const int i = q * 1024 + t;
+    rank[q] = 0;
+    if (q * 1024 + (t & ~63) >= R) continue;  // wave-uniform
+    const int e = i < R ? ids[i] : -1;
+    int c;
+    rank[q] = plan_wave_rank(e, ebits, c);
+    if (e >= 0 && rank[q] == 0) cnt[(i >> 6) * E + e] = c;
+  }
+  __syncthreads();
+  for (int e = t; e < E; e += 1024) {
+    int h = 0;
+    for (int g = 0; g < ngroup; g += 8) {
+      int c[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) c[j] = g + j < ngroup ? cnt[(g + j) * E + e] : 0;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        if (g + j < ngroup) cnt[(g + j) * E + e] = h;
+        h += c[j];
+      }
+    }
+    counts[e] = h;
+  }
+  __syncthreads();
+  if (t < 64) {
+    const int n = plan_offsets(E, counts, hist, offs, start);
+    if (t == 0) total = n;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int q = 0; q < kPlanSmallR / 1024; ++q) {
+    const int i = q * 1024 + t;
+    if (i >= R) continue;
+    const int e = ids[i];
+    if (e >= 0) {
+      const int pos = start[e] + cnt[(i >> 6) * E + e] + rank[q];
+      topk_indx[pos] = i;
+      gate_indx[i] = pos;
+      gate_scal[pos] = sc[i];
+    } else {
+      gate_indx[i] = -1;
+    }
+    if (i >= total) {  // slots past the valid entries
+      topk_indx[i] = -1;
+      gate_scal[i] = 0;
+    }
+  }
+  plan_maps(m, E, counts);
+}
+
+// ids and weights (MODE as above) and the expert counts of each chunk of kPlanTokens tokens: counts[chunk][E]
+template <int MODE>
+__global__ __launch_bounds__(1024) void token_hist_kernel(const uint16_t* __restrict__ logits, int64_t ld,
+                                                          const int32_t* __restrict__ idx, int64_t T, int E, int K,
+                                                          int32_t* __restrict__ ids, uint16_t* __restrict__ scal,
+                                                          int32_t* __restrict__ counts) {
+  __shared__ int32_t sh[kPlanMaxE];
+  const int t = threadIdx.x;
+  for (int e = t; e < E; e += 1024) sh[e] = 0;
+  __syncthreads();
+  const int64_t t0 = (int64_t)blockIdx.x * kPlanTokens;
+  if constexpr (MODE == 2) {
+    const int64_t hi = min((t0 + kPlanTokens) * K, T * K);
+    for (int64_t i = t0 * K + t; i < hi; i += 1024)
+      if (ids[i] >= 0) atomicAdd(&sh[ids[i]], 1);
+  } else {
+    for (int q = 0; q < kPlanTokens; q += 64) {
+      const int64_t tok = t0 + q + (t >> 4);
+      int32_t e;
+      uint16_t w;
+      plan_token<MODE == 0>(logits, ld, idx, tok, T, E, K, e, w);
+      if (tok < T && (t & 15) < K) {
+        ids[tok * K + (t & 15)] = e;
+        scal[tok * K + (t & 15)] = w;
+        if (e >= 0) atomicAdd(&sh[e], 1);
+      }
+    }
+  }
+  __syncthreads();
+  for (int e = t; e < E; e += 1024) counts[(int64_t)blockIdx.x * E + e] = sh[e];
+}
+
+// one block: counts[chunk][E] -> exclusive prefix over the chunks (in place), hist, offs, tile maps and orders
+__global__ __launch_bounds__(1024) void plan_scan_kernel(int32_t* __restrict__ counts, int n_chunks, int E, int epad,
+                                                         int32_t* __restrict__ hist, int32_t* __restrict__ offs,
+                                                         PlanMaps m) {
+  __shared__ int32_t cnt[kPlanMaxE];
+  __shared__ int32_t start[kPlanMaxE];
+  __shared__ int32_t seg_sum[1024];
+  // thread (seg, e): chunks [seg * per, (seg + 1) * per) of expert e
+  const int t = threadIdx.x, e = t & (epad - 1), seg = t / epad, nseg = 1024 / epad;
+  const int per = (n_chunks + nseg - 1) / nseg;
+  const int c0 = min(seg * per, n_chunks), c1 = e < E ? min(c0 + per, n_chunks) : c0;
+  auto load8 = [&](int c, int (&u)[8]) {
+#pragma unroll
+    for (int j = 0; j < 8; ++j) u[j] = counts[(int64_t)min(c + j, c1 - 1) * E + e];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) u[j] = c + j < c1 ? u[j] : 0;
+  };
+  int sum = 0;
+  for (int c = c0; c < c1; c += 8) {
+    int u[8];
+    load8(c, u);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) sum += u[j];
+  }
+  seg_sum[t] = sum;
+  __syncthreads();
+  int run = 0, all = 0;
+#pragma unroll 4
+  for (int s = 0; s < nseg; ++s) {
+    const int x = seg_sum[s * epad + e];
+    run += s < seg ? x : 0;
+    all += x;
+  }
+  for (int c = c0; c < c1; c += 8) {
+    int u[8];
+    load8(c, u);
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      if (c + j < c1) counts[(int64_t)(c + j) * E + e] = run;
+      run += u[j];
+    }
+  }
+  if (t < E) cnt[t] = all;  // threads 0 .. E - 1 are segment 0
+  __syncthreads();
+  if (t >= 960) plan_offsets(E, cnt, hist, offs, start);  // the last wave, the maps by the others
+  plan_maps(m, E, cnt);
+}
+
+// stable scatter of chunk blockIdx.x into expert-sorted order, and the slots past the valid entries
+__global__ __launch_bounds__(256) void plan_scatter_kernel(const int32_t* __restrict__ ids,
+                                                            const uint16_t* __restrict__ scal, int64_t R, int E, int K,
+                                                            int ebits, const int32_t* __restrict__ offs,
+                                                            const int32_t* __restrict__ counts,
+                                                            int32_t* __restrict__ topk_indx,
+                                                            int32_t* __restrict__ gate_indx,
+                                                            uint16_t* __restrict__ gate_scal) {
+  __shared__ int32_t base[kPlanMaxE];
+  __shared__ int32_t cnt[4 * kPlanMaxE];  // [wave][E] of one pass of 256 entries
+  const int t = threadIdx.x, wave = t >> 6;
+  for (int e = t; e < E; e += 256) base[e] = offs[e] + counts[(int64_t)blockIdx.x * E + e];
+  const int64_t valid = offs[E];
+  const int64_t lo = (int64_t)blockIdx.x * kPlanTokens * K;
+  const int64_t hi = min(lo + (int64_t)kPlanTokens * K, R);
+  for (int64_t i0 = lo; i0 < hi; i0 += 256) {
+    const int64_t i = i0 + t;
+    const int e = i < hi ? ids[i] : -1;
+    for (int q = t; q < 4 * E; q += 256) cnt[q] = 0;
+    __syncthreads();
+    int c;
+    const int rank = plan_wave_rank(e, ebits, c);
+    if (e >= 0 && rank == 0) cnt[wave * E + e] = c;
+    __syncthreads();
+    for (int x = t; x < E; x += 256) {
+      const int c0 = cnt[x], c1 = cnt[E + x], c2 = cnt[2 * E + x], c3 = cnt[3 * E + x], b0 = base[x];
+      cnt[x] = b0;
+      cnt[E + x] = b0 + c0;
+      cnt[2 * E + x] = b0 + c0 + c1;
+      cnt[3 * E + x] = b0 + c0 + c1 + c2;
+      base[x] = b0 + c0 + c1 + c2 + c3;
+    }
+    __syncthreads();
+    if (i < hi) {
+      if (e >= 0) {
+        const int pos = cnt[wave * E + e] + rank;
+        topk_indx[pos] = (int32_t)i;
+        gate_indx[i] = pos;
+        gate_scal[pos] = scal[i];
+      } else {
+        gate_indx[i] = -1;
+      }
+      if (i >= valid) {
+        topk_indx[i] = -1;
+        gate_scal[i] = 0;
+      }
+    }
+    __syncthreads();
+  }
+}
+
 // ---- expert data: padded tile offsets and block -> (block, expert) map -----
 // per tile size (one 1024-thread block each): the exclusive prefix of the
 // experts' tile counts -> offs_pad, then the tile -> (expert, tile) map
@@ -358,16 +825,76 @@ extern "C" size_t af3_routing_workspace_bytes(int64_t n_tokens, int n_expts_tot,
   return b + 256;
 }
 
+extern "C" size_t af3_routing_plan_workspace_bytes(int64_t n_tokens, int n_expts_tot, int n_expts_act, int topk);
+
+// whether the one-block plan takes the batch: replayed ids are one load per
+// slot, the top-k of more than a few passes of tokens goes over more blocks
+static bool plan_one_block(bool topk, int64_t T, int E, int K) {
+  const int64_t R = T * K;
+  return E <= kPlanMaxE && R <= kPlanSmallR && af3_cdiv(R, 64) * E <= kPlanSmallCnt &&
+         (!topk || E > kPlanMaxTopkE || T <= kPlanSmallTopkT);
+}
+
+// E <= 1024: the merged chain, with the tile maps of `m` where it asks for any
+static int routing_plan(bool topk, const uint16_t* logits, int64_t ld, const int32_t* expt_indx, int64_t T, int E, int K,
+                        uint16_t* gate_scal, int32_t* hist, int32_t* topk_indx, int32_t* gate_indx,
+                        int32_t* token_offs_raw, int32_t* ids, uint16_t* scal, int32_t* counts, const PlanMaps& m,
+                        hipStream_t stream) {
+  const int64_t R = T * K;
+  const int ebits = E > 1 ? 32 - __builtin_clz((unsigned)(E - 1)) : 1;
+  const bool lane_topk = topk && E <= kPlanMaxTopkE;
+  if (topk && !lane_topk && T > 0) {
+    hipLaunchKernelGGL(topk_token_kernel, dim3((unsigned)af3_cdiv(T, 128)), dim3(128), 0, stream, logits, ld, T, E, K,
+                       ids, scal);
+    int rc = af3::check_launch("routing/token");
+    if (rc) return rc;
+  }
+  const int mode = !topk ? 1 : lane_topk ? 0 : 2;
+  static_assert(kPlanSmallR <= kPlanSmallCnt && 2 * kPlanMaxBm <= 16, "the counters' other use; a wave per map and order");
+  if (plan_one_block(topk, T, E, K)) {
+#define AF3_PLAN(md)                                                                                                 \
+  hipLaunchKernelGGL(plan_small_kernel<md>, dim3(1), dim3(1024), 0, stream, logits, ld, expt_indx, (int)T, E, K, ids, \
+                     scal, ebits, gate_scal, hist, topk_indx, gate_indx, token_offs_raw, m)
+    if (mode == 0) AF3_PLAN(0);
+    else if (mode == 1) AF3_PLAN(1);
+    else AF3_PLAN(2);
+#undef AF3_PLAN
+    return af3::check_launch("routing/plan");
+  }
+  const int n_chunks = (int)af3_cdiv(T, kPlanTokens);
+#define AF3_TOK(md)                                                                                          \
+  hipLaunchKernelGGL(token_hist_kernel<md>, dim3(n_chunks), dim3(1024), 0, stream, logits, ld, expt_indx, T, E, K, \
+                     ids, scal, counts)
+  if (mode == 0) AF3_TOK(0);
+  else if (mode == 1) AF3_TOK(1);
+  else AF3_TOK(2);
+#undef AF3_TOK
+  int rc = af3::check_launch("routing/token_hist");
+  if (rc) return rc;
+  const int epad = 1 << ebits;  // >= E, <= 1024
+  hipLaunchKernelGGL(plan_scan_kernel, dim3(1), dim3(1024), 0, stream, counts, n_chunks, E, epad, hist, token_offs_raw,
+                     m);
+  rc = af3::check_launch("routing/scan");
+  if (rc) return rc;
+  hipLaunchKernelGGL(plan_scatter_kernel, dim3(n_chunks), dim3(256), 0, stream, ids, scal, R, E, K, ebits,
+                     token_offs_raw, counts, topk_indx, gate_indx, gate_scal);
+  return af3::check_launch("routing/scatter");
+}
+
 static int routing_common(bool topk, const uint16_t* logits, int64_t ld, const int32_t* expt_indx, int64_t T, int E,
                           int K, uint16_t* gate_scal, int32_t* hist, int32_t* topk_indx, int32_t* gate_indx,
-                          int32_t* token_offs_raw, void* workspace, size_t ws_bytes, hipStream_t stream) {
+                          int32_t* token_offs_raw, void* workspace, size_t ws_bytes, hipStream_t stream,
+                          const PlanMaps* maps = nullptr) {
   AF3_REQUIRE(T >= 0 && E > 0 && K > 0, "routing: bad sizes T=%lld E=%d K=%d", (long long)T, E, K);
   AF3_REQUIRE(K <= 16, "routing: K=%d > 16 unsupported", K);
   AF3_REQUIRE(E <= 0x7fff, "routing: E=%d too large", E);
   AF3_REQUIRE(E * 4 <= 48 * 1024, "routing: E=%d exceeds the per-chunk LDS histogram", E);
   AF3_REQUIRE(!topk || K <= E, "routing: K=%d > E=%d", K, E);
   AF3_REQUIRE(ld >= E, "routing: logits leading dim %lld < E", (long long)ld);
-  AF3_REQUIRE(ws_bytes >= af3_routing_workspace_bytes(T, E, K), "routing: workspace too small");
+  AF3_REQUIRE(ws_bytes >= (maps ? af3_routing_plan_workspace_bytes(T, E, K, topk)
+                                : af3_routing_workspace_bytes(T, E, K)),
+              "routing: workspace too small");
+  AF3_REQUIRE(!maps || E <= kPlanMaxE, "routing_plan: E=%d above %d", E, kPlanMaxE);
   const int64_t R = T * K;
   AF3_REQUIRE(R < 0x7fffffffLL, "routing: T*K too large");
   char* ws = (char*)workspace;
@@ -379,6 +906,11 @@ static int routing_common(bool topk, const uint16_t* logits, int64_t ld, const i
   o += (size_t)R * 2;
   o = (o + 255) & ~(size_t)255;
   int32_t* counts = (int32_t*)(ws + o);
+  if (E <= kPlanMaxE) {
+    const PlanMaps none{};
+    return routing_plan(topk, logits, ld, expt_indx, T, E, K, gate_scal, hist, topk_indx, gate_indx, token_offs_raw,
+                        ids, scal, counts, maps ? *maps : none, stream);
+  }
   const int n_chunks = (int)af3_cdiv(R, kChunk);
 
   if (T > 0) {
@@ -501,6 +1033,42 @@ extern "C" int af3_routing_topk(const uint16_t* logits, int64_t ld_logits, int64
                                 void* stream) {
   return routing_common(true, logits, ld_logits, nullptr, n_tokens, n_expts_tot, n_expts_act, gate_scal, hist,
                         topk_indx, gate_indx, token_offs_raw, workspace, ws_bytes, (hipStream_t)stream);
+}
+
+extern "C" size_t af3_routing_plan_workspace_bytes(int64_t n_tokens, int n_expts_tot, int n_expts_act, int topk) {
+  if (plan_one_block(topk != 0, n_tokens, n_expts_tot, n_expts_act) && !(topk && n_expts_tot > kPlanMaxTopkE)) return 0;
+  return af3_routing_workspace_bytes(n_tokens, n_expts_tot, n_expts_act);
+}
+
+// Routing and the grouped GEMM's tile metadata in one call (af3_routing_replay
+// / af3_routing_topk, then af3_expt_data and af3_tile_order per block size).
+extern "C" int af3_routing_plan(const uint16_t* logits, int64_t ld_logits, const int32_t* expt_indx, int topk,
+                                int64_t n_tokens, int n_expts_tot, int n_expts_act, uint16_t* gate_scal, int32_t* hist,
+                                int32_t* topk_indx, int32_t* gate_indx, int32_t* token_offs_raw, const int32_t* block_ms,
+                                int n_block_ms, int n_orders, int max_tiles, int32_t* token_offs_pad,
+                                int32_t* block_pid_map, int32_t* orders, void* workspace, size_t ws_bytes,
+                                void* stream) {
+  AF3_REQUIRE(block_ms && n_block_ms > 0 && n_block_ms <= kPlanMaxBm && n_orders >= 0 && n_orders <= n_block_ms &&
+                  max_tiles >= 0,
+              "routing_plan: bad block sizes (%d, %d orders, max_tiles %d)", n_block_ms, n_orders, max_tiles);
+  AF3_REQUIRE(n_expts_tot <= kPlanMaxE, "routing_plan: E=%d above %d", n_expts_tot, kPlanMaxE);
+  AF3_REQUIRE(token_offs_pad && (max_tiles == 0 || (block_pid_map && (n_orders == 0 || orders))),
+              "routing_plan: null pointer");
+  PlanMaps m{};
+  m.n_bm = n_block_ms;
+  m.n_order = n_orders;
+  m.max_tiles = max_tiles;
+  for (int i = 0; i < n_block_ms; ++i) {
+    AF3_REQUIRE(block_ms[i] > 0, "routing_plan: block size %d", block_ms[i]);
+    m.bm[i] = block_ms[i];
+  }
+  m.offs_pad = token_offs_pad;
+  m.map = block_pid_map;
+  m.order = orders;
+  AF3_REQUIRE(topk || expt_indx || n_tokens == 0, "routing_plan: null expt_indx");
+  return routing_common(topk != 0, logits, ld_logits, expt_indx, n_tokens, n_expts_tot, n_expts_act,
+                        gate_scal, hist, topk_indx, gate_indx, token_offs_raw, workspace, ws_bytes,
+                        (hipStream_t)stream, &m);
 }
 
 extern "C" int af3_expt_data(const int32_t* hist, int n_expts_tot, const int32_t* block_ms_dev, int n_block_ms,

@@ -94,6 +94,22 @@ int af3_routing_topk(const uint16_t* logits, int64_t ld_logits, int64_t n_tokens
                      int n_expts_act, uint16_t* gate_scal, int32_t* hist, int32_t* topk_indx, int32_t* gate_indx,
                      int32_t* token_offs_raw, void* workspace, size_t ws_bytes, void* stream);
 
+/* Routing (topk != 0: af3_routing_topk, else af3_routing_replay) and the tile
+ * metadata of its result (af3_expt_data for every size of the host array
+ * block_ms, af3_tile_order for the first n_orders of them) in one call: one
+ * launch for small batches, three otherwise.  token_offs_pad [n_block_ms][E+1],
+ * block_pid_map [n_block_ms][max_tiles], orders [n_orders][max_tiles], all -1
+ * past each size's tiles; E <= 1024, n_block_ms <= 8.  The workspace is
+ * af3_routing_plan_workspace_bytes (0 for the one-launch form).  No counterpart
+ * in the reference, which makes these tensors one torch op at a time
+ * (quantization.py:593-636). */
+size_t af3_routing_plan_workspace_bytes(int64_t n_tokens, int n_expts_tot, int n_expts_act, int topk);
+int af3_routing_plan(const uint16_t* logits, int64_t ld_logits, const int32_t* expt_indx, int topk, int64_t n_tokens,
+                     int n_expts_tot, int n_expts_act, uint16_t* gate_scal, int32_t* hist, int32_t* topk_indx,
+                     int32_t* gate_indx, int32_t* token_offs_raw, const int32_t* block_ms, int n_block_ms, int n_orders,
+                     int max_tiles, int32_t* token_offs_pad, int32_t* block_pid_map, int32_t* orders, void* workspace,
+                     size_t ws_bytes, void* stream);
+
 /* Router logits.  Replaces nn.functional.linear(hidden_states,
  * router.weight, router.bias) in mlp_forward (quantization.py:653-654):
  * logits[t][e] = bf16(sum_k x[t][k] w[e][k] + bias[e]) with fp32 sums.
