@@ -64,7 +64,18 @@ GEMM_BLOCK_M = 128
 # the 256 x 256 kernels (tile_cfg 22 / 23).  The LoRA row products always use
 # the 128-row map.  x_off32: tell the library when x lies within 4 GiB (the
 # forward then addresses it by a scalar base and 32-bit offsets).
-GEMM_TILE = {"block_m": 256, "tile_cfg": 0, "fwd_block_m": 128, "dx_block_m": 128}
+# With few rows per expert (routed rows <= the limit times the experts) they take
+# the 32- or 64-row map and the short-tile kernels (tile_cfg 27 / 29) instead.
+# Measured, both launches of a 120b layer (E 128, top-4, rank 32), us, 128- /
+# 32- / 64-row map: forward 301 tokens (9 rows per expert) 409 / 354 / 361, 600
+# (19) 421 / 373 / 377, 1021 (32) 460 / 537 / 422, 1500 (47) 488 / 731 / 465,
+# under Zipf loads 600 441 / 404 / 408, 1500 551 / 562 / 531; input gradient 40
+# (1) 345 / 294 / 338, 301 420 / 382 / 398, 600 437 / 400 / 416, 1021 467 / 601 /
+# 449, 1500 513 / 993 / 620, Zipf 400 438 / 422 / 446, 600 454 / 491 / 470, 1021
+# 555 / 552 / 527.
+GEMM_TILE = {"block_m": 256, "tile_cfg": 0, "fwd_block_m": 128, "dx_block_m": 128, "short": True}
+FWD_SHORT_ROWS = ((24, 32), (48, 64))   # (rows per expert at most, block_m)
+DX_SHORT_ROWS = ((13, 32), (32, 64))
 
 # The expert module's forward GEMMs read a tiled copy of each frozen
 # projection's packed weights (af3_mxfp4_tile_fwd: the words one k-step of a
@@ -250,6 +261,19 @@ def mxfp4_tile_dx_scales(scales):
     return out
 
 
+def _short_block_m(ed, rows, E, N, K, trans_w, off32):
+    """The short-tile kernels' map (32 or 64 rows) for a launch of ``rows`` rows
+    over E experts, or 0: they need few rows per expert, the map (made with the
+    routing), 32-bit offsets, and whole 320-deep (forward) k-groups."""
+    if not GEMM_TILE.get("short", True) or not off32 or N % 64 or N * K // 2 >= 1 << 32 \
+            or (not trans_w and (K % 320 or K > 3072)):
+        return 0
+    for lim, bm in DX_SHORT_ROWS if trans_w else FWD_SHORT_ROWS:
+        if rows <= lim * E and bm in ed.block_pid_map and bm in ed.gemm_order:
+            return bm
+    return 0
+
+
 def moe_rows(x, blocks, scales, bias, routing_data, gather_indx=None, gammas=None, trans_w=False,
              lora_l=None, lora_b=None, swiglu=None, a_row_scale=None, w_tiled=None, s_tiled=None):
     """Expert-sorted output rows of the grouped GEMM (no scatter).
@@ -284,6 +308,9 @@ def moe_rows(x, blocks, scales, bias, routing_data, gather_indx=None, gammas=Non
     R = g.shape[0] if g is not None else x.shape[0]
     routing_data, k_act = _expt_data(routing_data, R, dev)
     ed = routing_data.expt_data
+    ldx = x.stride(0) if x.shape[0] > 1 else K
+    # every row of x lies within 4 GiB of x: the kernels may address it by 32-bit offsets
+    off32 = GEMM_TILE.get("x_off32", True) and ((x.shape[0] - 1) * ldx + K) * 2 <= 1 << 32
     bm = GEMM_TILE["block_m"] if K % 64 == 0 else 128
     if K % 64 == 0 and a_row_scale is None:
         # the default kernels (tile_cfg 26 forward, 28 input gradient) run on the 128-row map
@@ -291,6 +318,8 @@ def moe_rows(x, blocks, scales, bias, routing_data, gather_indx=None, gammas=Non
             bm = GEMM_TILE.get("fwd_block_m", 128)
         elif trans_w and GEMM_TILE["tile_cfg"] % 100 in (0, 28):
             bm = GEMM_TILE.get("dx_block_m", 128)
+        if GEMM_TILE["tile_cfg"] == 0 and bm == 128:
+            bm = _short_block_m(ed, R, E, N, K, trans_w, off32) or bm
     pid_map = gemm_order_for(ed, bm) if GEMM_TILE.get("order", True) else None
     if pid_map is None:
         pid_map = ed.block_pid_map[bm]
@@ -332,9 +361,6 @@ def moe_rows(x, blocks, scales, bias, routing_data, gather_indx=None, gammas=Non
         lr = lora_l.shape[-1]
         lora_l = lora_l.contiguous()
         lora_b = lora_b.to(torch.bfloat16).contiguous()
-    ldx = x.stride(0) if x.shape[0] > 1 else K
-    # every row of x lies within 4 GiB of x: the kernels may address it by 32-bit offsets
-    off32 = GEMM_TILE.get("x_off32", True) and ((x.shape[0] - 1) * ldx + K) * 2 <= 1 << 32
     cfg = GEMM_TILE["tile_cfg"] | (_capi.X_OFFSETS_32 if off32 else 0)
     args = (x.data_ptr(), ldx, _capi.ptr(g), k_act if g is not None else 1,
             blocks.data_ptr(), scales.data_ptr(), 1 if trans_w else 0, _capi.ptr(b), _capi.ptr(gm), gm_f32,
@@ -351,11 +377,11 @@ def moe_rows(x, blocks, scales, bias, routing_data, gather_indx=None, gammas=Non
     # the default input-gradient kernel; any other selection declines them
     # (nothing launched) and the stored blocks / scales are used
     targs = None
-    if w_tiled is not None and not trans_w and a_row_scale is None and bm == 128 \
+    if w_tiled is not None and not trans_w and a_row_scale is None and bm <= 128 \
             and GEMM_TILE["tile_cfg"] % 100 in (0, 26):
         targs = list(args)
         targs[4], targs[19] = w_tiled.data_ptr(), cfg | _capi.W_FWD_TILED
-    if s_tiled is not None and trans_w and a_row_scale is None and bm == 128 \
+    if s_tiled is not None and trans_w and a_row_scale is None and bm <= 128 \
             and GEMM_TILE["tile_cfg"] % 100 in (0, 28):
         if s_tiled.dtype != torch.uint8 or not s_tiled.is_contiguous() \
                 or s_tiled.numel() != E * ((N + 255) // 256) * ((K // 64) * 512 + 1):

@@ -621,6 +621,25 @@ static inline unsigned g4_grid(int max_tiles, int NN, int GM) {
   return (unsigned)(8 * ((groups + 7) / 8) * GM * NN);
 }
 
+// Work item of the short-tile kernels (32 / 64-row maps) when there are fewer
+// than kG9SpreadTiles m-tiles: the unit dealt to the XCDs in turn is GM m-tiles
+// x one n-tile.  Dealing whole groups of n-tiles as g4_work_item does would
+// leave XCDs idle then (one token: 4 m-tiles, two groups).
+__device__ __forceinline__ bool g9_work_item(const Params& p, int& mt, int& nt) {
+  const int NN = p.n_nblk, Mt = p.tile_offs[p.E], GM = p.group_m;
+  const int x = blockIdx.x & 7, j = blockIdx.x >> 3;
+  const int u = x + 8 * (j / GM);
+  nt = u % NN;
+  mt = (u / NN) * GM + j % GM;
+  return mt < Mt;
+}
+
+constexpr int kG9SpreadTiles = 16;  // fewer m-tiles than this: the spread order
+static inline unsigned g9_grid(int max_tiles, int NN, int GM) {
+  const long long units = (long long)((max_tiles + GM - 1) / GM) * NN;
+  return (unsigned)(8 * ((units + 7) / 8) * GM);
+}
+
 // Epilogue of a 256x256 (or CN = 512: 128x512) tile computed by waves of 32x32 MFMA
 // sub-tiles: v = (acc + bias[n]) * gamma[row] -> bf16, staged through LDS as
 // a [256][256] bf16 tile (16-byte chunks XOR-swizzled so the two row groups
@@ -873,29 +892,34 @@ __device__ __forceinline__ void g7_landed(af3_u32x4 (&r)[TN]) {
 // <= 128 rows converts each weight byte once per 128 rows instead of per 256).
 // The 8 waves are WM x WN (NARROW: 1 x 8) of the same 128 x 64 wave tile.
 // SHAPE 0: 256 x 256 (WM x WN waves), 1 (NARROW): 128 x 512 (8 waves side by
-// side), 2 (HALF): 128 x 256 (4 waves side by side; two blocks per CU)
+// side), 2 (HALF): 128 x 256 (4 waves side by side; two blocks per CU), 3 / 4
+// (SKINNY): 32 / 64 x 256 on the 32 / 64-row map, NB weight buffers and as many
+// A stages, so NB - 1 k-steps are in flight
 template <int WM, int WN, int BXK, int SHAPE, bool BG = false, int NB = 2, bool SA = false>
 __device__ __forceinline__ void g4f_tile(const Params& p, uint8_t* lds, int e, int row_lo, int nrows, int n0,
                                          int ncols) {
-  constexpr bool NARROW = SHAPE == 1, HALF = SHAPE == 2;
-  static_assert(NB == 2 || (NB == 3 && BG), "weight register buffers: 2, or 3 (BG, k-steps a multiple of 3)");
+  constexpr bool NARROW = SHAPE == 1, SKINNY = SHAPE >= 3, HALF = SHAPE == 2 || SKINNY;
+  static_assert(NB == 2 || (NB == 3 && BG) || (SKINNY && NB >= 3),
+                "weight register buffers: 2, or more where the k-steps are a multiple of them");
+  constexpr int ST = SKINNY ? NB : kG4Stages;  // A stages
   // SA (BG): the k-loop's A copies and weight loads address a scalar base
   // plus a 32-bit per-lane offset (a_off32; the expert's packed weights < 4 GiB)
   static_assert(!SA || BG, "scalar-base addressing in the register-weight kernel");
   static_assert(!HALF || BG, "the 128 x 256 shape takes the packed weights from registers");
   constexpr int NW = HALF ? 4 : WM * WN, NT = NW * 64;
-  constexpr int RM = (NARROW || HALF) ? 128 : kG4Rows, CN = NARROW ? 512 : kG4Rows;
+  constexpr int RM = SHAPE == 3 ? 32 : SHAPE == 4 ? 64 : (NARROW || HALF) ? 128 : kG4Rows, CN = NARROW ? 512 : kG4Rows;
   constexpr int WMX = (NARROW || HALF) ? 1 : WM, WNX = (NARROW || HALF) ? NW : WN;
   constexpr int TM = RM / WMX / 32, TN = CN / WNX / 32;
   constexpr int ASTAGE = RM * kBK;  // bf16 elements per A stage
   constexpr int BSTAGE = CN * 32;   // bytes per packed-B stage
   // copies per wave per k-step (BG: the packed weights go straight to registers, no B copies)
   constexpr int API = RM / 8 / NW, BPI = BG ? 0 : CN / 32 / NW, DPW = API + BPI;
-  static_assert(API >= 1 && (BG || BPI >= 1) && (DPW == 10 || DPW == 8 || DPW == 5 || DPW == 4 || DPW == 2),
+  static_assert(API >= 1 && (BG || BPI >= 1) && (DPW == 10 || DPW == 8 || DPW == 5 || DPW == 4 || DPW == 2 ||
+                                                     (SKINNY && DPW == 1)),
                 "copy schedule");
-  static_assert(kG4Stages * (ASTAGE * 2 + BSTAGE) <= kG4Stages * (kG4AStage * 2 + kG4BStage), "LDS ring");
-  uint16_t* const As = (uint16_t*)lds;                    // 3 x RM x 64 bf16
-  uint8_t* const Bs = lds + kG4Stages * ASTAGE * 2;       // 3 x CN x 32 bytes (not with BG)
+  static_assert(SKINNY || kG4Stages * (ASTAGE * 2 + BSTAGE) <= kG4Stages * (kG4AStage * 2 + kG4BStage), "LDS ring");
+  uint16_t* const As = (uint16_t*)lds;                    // ST x RM x 64 bf16
+  uint8_t* const Bs = lds + ST * ASTAGE * 2;              // 3 x CN x 32 bytes (not with BG)
   uint8_t* const Ss = BG ? Bs : Bs + kG4Stages * BSTAGE;  // CN x G scale bytes
   const int G = p.K >> 5;
   const int nk = p.K / kBK;
@@ -945,7 +969,7 @@ __device__ __forceinline__ void g4f_tile(const Params& p, uint8_t* lds, int e, i
   // copy j (0..DPW-1) of k-step kt: API A instructions (8 rows each), then BPI packed-B
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_addr(lds));  // LDS byte address of the block's area
   auto issue_one = [&](int kt, int j) {
-    const int st = kt % kG4Stages;
+    const int st = kt % ST;
     // BG: the k-steps past the end copy the last k-step's rows again (into a stage no wave reads again)
     const int ks = BG ? min(kt, nk - 1) : kt;
     if (j < API) {
@@ -1028,18 +1052,24 @@ __device__ __forceinline__ void g4f_tile(const Params& p, uint8_t* lds, int e, i
 
   // two blocks share each CU: while one runs its epilogue (VALU and memory
   // work), the other's k-loop keeps issue priority for its MFMAs and copies
-  if constexpr (HALF) __builtin_amdgcn_s_setprio(2);
+  if constexpr (HALF && !SKINNY) __builtin_amdgcn_s_setprio(2);
   // BG: the weight words of k-step 0 (NB = 3: and 1), each before its
   // k-step's copies (the order every later k-step keeps: its weight loads
   // first, then its copies)
-  if constexpr (BG) {
+  if constexpr (SKINNY) {
+    // after the scale check, in the compiled k-loop it chooses: no branch lies
+    // between these loads and the loop, so no register of a load in flight is
+    // copied at a join
+  } else if constexpr (BG) {
     if (live) load_b(0, std::integral_constant<int, 0>{});
   }
-  issue(0);
-  if constexpr (NB == 3) {
-    if (live) load_b(1, std::integral_constant<int, 1>{});
+  if constexpr (!SKINNY) {
+    issue(0);
+    if constexpr (NB == 3) {
+      if (live) load_b(1, std::integral_constant<int, 1>{});
+    }
+    if (BG || nk > 1) issue(1);
   }
-  if (BG || nk > 1) issue(1);
   // does the tile hold a scale byte outside [2, 252]?  (then the whole work
   // item takes the exact integer dequantisation)
   bool odd = false;
@@ -1065,6 +1095,17 @@ __device__ __forceinline__ void g4f_tile(const Params& p, uint8_t* lds, int e, i
     constexpr bool FULL = decltype(full_c)::value, EXACT = decltype(exact_c)::value;
     constexpr int TMV = decltype(rows_c)::value;
     static_assert(FULL || TMV == TM, "run-time sub-tile selection covers all row groups");
+    if constexpr (SKINNY) {  // k-steps 0 .. NB - 2: each one's weight loads, then its copies
+      auto pro = [&](auto k) {
+        load_b(decltype(k)::value, k);
+        issue(decltype(k)::value);
+      };
+      pro(std::integral_constant<int, 0>{});
+      pro(std::integral_constant<int, 1>{});
+      if constexpr (NB > 3) pro(std::integral_constant<int, 2>{});
+      if constexpr (NB > 4) pro(std::integral_constant<int, 3>{});
+      static_assert(NB <= 5, "prologue");
+    }
     af3_bf16x8 af[2][TMV], bf[2][TN];
     const af3_bf16x8 zf = __builtin_bit_cast(af3_bf16x8, zero4());
 #pragma unroll
@@ -1085,7 +1126,10 @@ __device__ __forceinline__ void g4f_tile(const Params& p, uint8_t* lds, int e, i
         // NB - 1 k-steps later) and then API copies (for two k-steps later), so
         // this k-step's data is everything but the newest API operations (NB =
         // 2) or the newest TN + API (NB = 3: the previous k-step's loads too)
-        if constexpr (NB == 3) {
+        if constexpr (SKINNY) {
+          // in flight past this k-step's: the NB - 2 newer k-steps' loads and copies
+          asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NB - 2) * (TN + DPW)) : "memory");
+        } else if constexpr (NB == 3) {
           static_assert(DPW + TN == 6, "wait count");
           AF3_ASM_WAIT_VM(6);
         } else {
@@ -1098,7 +1142,7 @@ __device__ __forceinline__ void g4f_tile(const Params& p, uint8_t* lds, int e, i
         wait_stage(last);
         AF3_ASM_LDS_BARRIER();
       }
-      const int st = kt % kG4Stages;
+      const int st = kt % ST;
       g4_kstep<TMV, TN, DPW, FULL, EXACT, BG>(As + st * ASTAGE, Bs + st * BSTAGE, bq[P], Ss, G, kt, BG || !last,
                                               wm0, wn0, tm_live, tn_live, acc, af, bf, sc, dma);
     };
@@ -1108,7 +1152,16 @@ __device__ __forceinline__ void g4f_tile(const Params& p, uint8_t* lds, int e, i
     constexpr std::true_type LAST{};
     int kt = 0;
     if constexpr (BG) {
-      if constexpr (NB == 3) {
+      if constexpr (SKINNY) {
+        // whole groups of NB k-steps (nk % NB == 0)
+        for (; kt < nk; kt += NB) {
+          step(kt, MORE, I0, [&](int j) { issue_one(kt + NB - 1, j); });
+          step(kt + 1, MORE, I1, [&](int j) { issue_one(kt + NB, j); });
+          step(kt + 2, MORE, std::integral_constant<int, 2>{}, [&](int j) { issue_one(kt + NB + 1, j); });
+          if constexpr (NB > 3) step(kt + 3, MORE, std::integral_constant<int, 3>{}, [&](int j) { issue_one(kt + NB + 2, j); });
+          if constexpr (NB > 4) step(kt + 4, MORE, std::integral_constant<int, 4>{}, [&](int j) { issue_one(kt + NB + 3, j); });
+        }
+      } else if constexpr (NB == 3) {
         // whole triples (nk % 3 == 0; the register buffer of each k-step is
         // static and no path of the compiled loop skips a k-step)
         for (; kt < nk; kt += 3) {
@@ -1157,9 +1210,17 @@ __device__ __forceinline__ void g4f_tile(const Params& p, uint8_t* lds, int e, i
         kloop(std::true_type{}, exact_c, std::integral_constant<int, 2>{});
       else
         kloop(std::true_type{}, exact_c, std::integral_constant<int, 1>{});
+    } else if constexpr (SKINNY) {
+      if constexpr (TM == 2) {
+        if (tm_live == 1) {
+          kloop(std::true_type{}, exact_c, std::integral_constant<int, 1>{});
+          return;
+        }
+      }
+      kloop(std::true_type{}, exact_c, ALL_ROWS);
     }
   };
-  if (NB == 3 && tm_live > 0 && tn_live > 0) {
+  if (NB >= 3 && tm_live > 0 && tn_live > 0) {
     if (odd)
       by_rows(std::true_type{});
     else
@@ -1183,8 +1244,16 @@ __device__ __forceinline__ void g4f_tile(const Params& p, uint8_t* lds, int e, i
     // a wave with no live sub-tile (rows or columns past the end of a
     // partial tile) only keeps the copy / barrier protocol of the k-loop, so
     // the live wave sharing its SIMD runs alone
+    if constexpr (SKINNY) {
+#pragma unroll
+      for (int k = 0; k < NB - 1; ++k) issue(k);
+    }
     for (int kt = 0; kt < nk; ++kt) {
-      if constexpr (BG) {
+      if constexpr (SKINNY) {
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NB - 2) * DPW) : "memory");
+        AF3_ASM_LDS_BARRIER();
+        issue(kt + NB - 1);
+      } else if constexpr (BG) {
         wait_stage(false);
         AF3_ASM_LDS_BARRIER();
         issue(kt + 2);
@@ -1215,7 +1284,7 @@ __device__ __forceinline__ void g4f_tile(const Params& p, uint8_t* lds, int e, i
     }
   }
 
-  if constexpr (HALF) __builtin_amdgcn_s_setprio(0);  // the k-loop's waves first (see the k-loop's start)
+  if constexpr (HALF && !SKINNY) __builtin_amdgcn_s_setprio(0);  // the k-loop's waves first (see the k-loop's start)
   g4_epilogue<false, TM, TN, NT, CN, RM>(p, lds, acc, e, row_lo, nrows, n0, ncols, wm0, wn0);
 }
 
@@ -1265,6 +1334,37 @@ __global__ __launch_bounds__(256, 2) void gemm7_fwd_kernel(Params p) {
   if (nrows <= 0) return;
   const int n0 = nt * 256;
   g4f_tile<1, 4, BXK, 2, true, NB, SA>(p, lds, e, row_lo, nrows, n0, min(256, p.N - n0));
+}
+
+// Short expert tiles (few rows per expert): RM x 256 items on the RM-row map,
+// RM = 32 / 64.  The launch reads every live expert's weights once and is bound
+// by that stream; gemm7 on such a tile copies all 128 A rows per k-step (twice
+// the weight bytes, mostly repeats of row 0) and keeps two k-steps of weights
+// in flight on two blocks per CU.  Here a k-step copies RM rows, four k-steps
+// are in flight (weights in five register buffers, A in five LDS stages) and
+// three (RM 64: two) blocks share a CU.  Same fragments and sums as gemm7.
+// Measured (both launches of a forward): 301 tokens over 128 experts, rank 32,
+// 409 -> 354 us (1.73 GB, 4.9 TB/s), 1021 tokens 460 -> 422 (64 rows), 23
+// tokens over 32 experts 131 -> 103, one token 72 -> 52.
+constexpr int kG9NB = 5;
+template <int RM>
+constexpr int kG9LdsBytes = kG9NB * RM * kBK * 2 + 256 * kG7MaxG;  // 44 / 64 KB
+static_assert(kG9LdsBytes<32> >= (32 + 256) * kBK * 2 && kG9LdsBytes<64> >= (64 + 256) * kBK * 2, "LoRA segment");
+static_assert(kG9LdsBytes<32> >= 32 * 520 && kG9LdsBytes<64> >= 64 * 520, "epilogue");
+
+template <int BXK, int RM>
+__global__ __launch_bounds__(256, RM == 32 ? 3 : 2) void gemm9_fwd_kernel(Params p) {
+  __shared__ __attribute__((aligned(16))) uint8_t lds[kG9LdsBytes<RM>];
+  int mt, nt;
+  if (!(p.tile_offs[p.E] < kG9SpreadTiles ? g9_work_item(p, mt, nt) : g4_work_item(p, mt, nt))) return;
+  const int32_t ent = p.tile_map[mt];
+  if (ent < 0) return;
+  const int e = ent & 0xFFFF, blk = ent >> 16;
+  const int row_lo = p.offs[e] + blk * RM;
+  const int nrows = min(RM, p.offs[e + 1] - row_lo);
+  if (nrows <= 0) return;
+  const int n0 = nt * 256;
+  g4f_tile<1, 4, BXK, RM == 32 ? 3 : 4, true, kG9NB, true>(p, lds, e, row_lo, nrows, n0, min(256, p.N - n0));
 }
 
 // ---------------------------------------------------------------------------
@@ -1693,13 +1793,16 @@ __device__ __forceinline__ void d5_epilogue(const Params& p, uint8_t* lds, af3_f
 // blocks x 64 rows of a k-step are 128 contiguous bytes, taken by one 2-byte
 // copy per lane (rows 2 l, 2 l + 1 of block l / 32 in lane l's LDS dword)
 // instead of two 1-byte copies that read 64 rows each.
-template <bool NARROW, int BXK, int SPLIT = 1, int RG = 0, bool HALF = false, bool SADDR = false, bool TS = false>
+// RMH: rows of a HALF item (128; 32 / 64 on the 32 / 64-row maps).
+template <bool NARROW, int BXK, int SPLIT = 1, int RG = 0, bool HALF = false, bool SADDR = false, bool TS = false,
+          int RMH = 128>
 __device__ __forceinline__ void d5_tile(const Params& p, uint8_t* lds, int e, int row_lo, int nrows, int n0, int ncols) {
   static_assert(!(NARROW && HALF), "one item shape");
   static_assert(!TS || HALF, "tiled input-gradient scales on the 128 x 256 items");
   static_assert(SPLIT == 1 || (!NARROW && !HALF && (SPLIT == 2 || SPLIT == 4)), "row split only for 256-row tiles");
   static_assert(RG == 0 || (SPLIT == 1 && RG >= 1 && RG <= ((NARROW || HALF) ? 4 : 8)), "row groups of a tile");
-  constexpr int RM = (NARROW || HALF) ? 128 : 256;  // tile rows
+  static_assert(RMH == 128 || (HALF && (RMH == 32 || RMH == 64)), "rows of a HALF item");
+  constexpr int RM = HALF ? RMH : NARROW ? 128 : 256;  // tile rows
   constexpr int CN = NARROW ? 512 : 256;  // tile columns
   constexpr int TM = RM / 32;             // row groups of the tile
   constexpr int TMW = RG ? RG : TM / SPLIT;  // row groups of one wave
@@ -1710,10 +1813,10 @@ __device__ __forceinline__ void d5_tile(const Params& p, uint8_t* lds, int e, in
   constexpr int NCH = BRB / 16;           // 16-byte chunks per weight row
   constexpr int NBLK = CN / 32;           // scale blocks
   constexpr int AI = RM / 32, BI = BRB / 64, SI = NBLK / 4;  // copies per wave per k-step
-  constexpr int NCP = AI + BI + SI;
-  static_assert(NCP == (HALF ? 8 : 12), "12 (HALF: 8) copies per wave per k-step");
-  constexpr int AOFF = 0, BOFF = (NARROW || HALF) ? 16384 : 32768, SOFF = NARROW ? 32768 : HALF ? 24576 : 40960;
-  constexpr int STAGE = HALF ? kD5HStage : kD5Stage;
+  constexpr int NCP = AI + BI + (TS ? 1 : SI);
+  static_assert(NCP == (HALF ? RMH / 32 + (TS ? 3 : 4) : 12), "copies per wave per k-step");
+  constexpr int AOFF = 0, BOFF = RM * 128, SOFF = BOFF + 64 * BRB;
+  constexpr int STAGE = HALF ? RMH * 128 + 64 * 128 + 8 * 64 * 4 : kD5Stage;
   static_assert(SOFF + NBLK * 256 <= STAGE, "stage layout");
   // slot of chunk c in weight row k (keeps the transposing reads conflict-free)
   auto bswz = [](int k) { return NARROW ? ((k & 7) << 1) : (k & 7); };
@@ -1766,9 +1869,9 @@ __device__ __forceinline__ void d5_tile(const Params& p, uint8_t* lds, int e, in
   const uint8_t* const tsb = p.b.scales + ((int64_t)e * nk * p.s_nt + (n0 >> 8)) * 512 + wave * 128;
   const int64_t tstep = (int64_t)p.s_nt * 512;
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane(lds_addr(lds));
-  // copy j (0..11) of k-step kc: A, then B, then S (TS: one S copy, j = AI + BI)
-  auto issue_one = [&](int kc, int j) {
-    const uint32_t st = lds0 + (uint32_t)((kc % kD5Stages) * STAGE);
+  // copy j of k-step kc into the stage at LDS byte offset so: A, then B, then S (TS: one S copy, j = AI + BI)
+  auto issue_one = [&](int kc, uint32_t so, int j) {
+    const uint32_t st = lds0 + so;
     if (j < AI) {
       const uint32_t dst = st + (uint32_t)(AOFF + (wave * AI + j) * 1024);
       if constexpr (SADDR)
@@ -1794,10 +1897,11 @@ __device__ __forceinline__ void d5_tile(const Params& p, uint8_t* lds, int e, in
         asm volatile("s_nop 0\n\tglobal_load_lds_ubyte %0, off" ::"v"(ssrc[j - AI - BI] + kc * sstep), "{m0}"(dst) : "memory");
     }
   };
-  auto issue = [&](int kc) {
+  auto issue_from = [&](int kc, uint32_t so) {
 #pragma unroll
-    for (int j = 0; j < NCP; ++j) issue_one(kc, j);
+    for (int j = 0; j < NCP; ++j) issue_one(kc, so, j);
   };
+  auto issue = [&](int kc) { issue_from(kc, (uint32_t)(kc * STAGE)); };
 
   // ---- lane-fixed LDS byte offsets inside a stage ----
   const int ax = (lr ^ (lr >> 3)) & 7;
@@ -1837,7 +1941,7 @@ __device__ __forceinline__ void d5_tile(const Params& p, uint8_t* lds, int e, in
   // work), the other's k-loop keeps issue priority for its MFMAs and copies
   if constexpr (HALF) __builtin_amdgcn_s_setprio(2);
   issue(0);
-  if (nk > 1) issue(1);
+  issue_from(min(1, nk - 1), STAGE);
 
   // TS: the exact conversion is chosen per work item (the tiled scales carry a
   // flag per expert and n-tile: any scale byte outside [2, 252]), so the
@@ -1847,12 +1951,22 @@ __device__ __forceinline__ void d5_tile(const Params& p, uint8_t* lds, int e, in
     constexpr bool FULL = decltype(full_c)::value;
     constexpr int XC = decltype(exact_c)::value;  // 0: never exact, 1: always, 2: per k-step check
     af3_bf16x8 af[2][TMW], bf[2][TN];
+    // The k-loop is bound by instruction issue (44% of the waves' cycles issue),
+    // so nothing but the data path is in it: scale bytes take one shift (the
+    // conversion ignores sign and mantissa), the ring's stage offsets are carried
+    // scalars, copies and waits are unconditional.  223 instructions per k-step
+    // of the tiled-scale 128 x 256 item against 306 with masks, a modulo per LDS
+    // address and guarded copies; a 20b layer's two launches (16384 tokens) 3163
+    // -> 3020 us.
     // one k-step: iterations s = -1 (the carried sub-step of the previous
     // k-step, skipped at kt = 0) and 0..2; iteration s runs the MFMAs of
     // sub-step s while reading and converting the fragments of s + 1
-    auto kstep = [&](int kt, bool first, bool pf) {
-      const uint8_t* stg = lds + (kt % kD5Stages) * STAGE;
-      const int nxt_copy = kt + 2;
+    // so: the k-step's stage (LDS byte offset), nso: the one its copies (for kt + 2) go to
+    // (uniform k-steps: the last two copy the last k-step again, into stages no
+    // wave reads again, so no copy and no wait of the loop is conditional)
+    auto kstep = [&](int kt, uint32_t so, uint32_t nso, bool first) {
+      const uint8_t* stg = lds + so;
+      const int nxt_copy = min(kt + 2, nk - 1);
       bool odd = false;
 #pragma unroll
       for (int s = -1; s < 3; ++s) {
@@ -1860,7 +1974,7 @@ __device__ __forceinline__ void d5_tile(const Params& p, uint8_t* lds, int e, in
         const int nx = s < 0 ? 0 : (c ^ 1);  // fragments of sub-step s + 1
         const int o = s + 1;                 // sub-step whose operands are read
         uint32_t w[PG][2];
-        uint32_t sc[PG][8];
+        uint32_t sc[PG][8];  // scale operands: the byte at the exponent's place
         uint32_t chk[CW];
 #pragma unroll
         for (int q = 0; q < CW; ++q) chk[q] = 2;
@@ -1893,19 +2007,20 @@ __device__ __forceinline__ void d5_tile(const Params& p, uint8_t* lds, int e, in
               w[pg][1] = (uint32_t)wv[1];
             } else if (i < SC) {
               const int pg = (i - SB) >> 1, h = (i - SB) & 1;
-              if constexpr (TS) {  // 4 dwords = the 8 rows' bytes, two per dword
+              if constexpr (TS) {  // 4 dwords = the 8 rows' bytes, two per dword (one shift each: the
+                                   // conversion reads only the exponent field, whatever the others hold)
                 if (h == 0) {
                   const af3_u32x4 sv = *(const af3_u32x4*)(stg + soff[pg] + 16 * o);
 #pragma unroll
                   for (int q = 0; q < 4; ++q) {
-                    sc[pg][2 * q] = sv[q] & 0xFFu;
-                    sc[pg][2 * q + 1] = (sv[q] >> 8) & 0xFFu;
+                    sc[pg][2 * q] = sv[q] << 23;
+                    sc[pg][2 * q + 1] = sv[q] << 15;
                   }
                 }
               } else {
                 const af3_u32x4 sv = *(const af3_u32x4*)(stg + soff[pg] + 32 * o + 16 * h);
 #pragma unroll
-                for (int q = 0; q < 4; ++q) sc[pg][4 * h + q] = sv[q];
+                for (int q = 0; q < 4; ++q) sc[pg][4 * h + q] = sv[q] << 23;
               }
             } else if (i == SC) {
               if (s < 0 && XC == 2) {
@@ -1933,7 +2048,7 @@ __device__ __forceinline__ void d5_tile(const Params& p, uint8_t* lds, int e, in
               if (i >= c0 && i < c0 + 8 && (FULL || pg < pg_live)) {
                 const int q = i - c0;
                 const uint32_t src = w[pg][q >> 2];
-                const float scf = __uint_as_float(sc[pg][q] << 23);
+                const float scf = __uint_as_float(sc[pg][q]);
                 switch (q & 3) {
                   case 0: dw[pg][q] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(src, scf, 0)); break;
                   case 1: dw[pg][q] = __builtin_bit_cast(uint32_t, __builtin_amdgcn_cvt_scalef32_pk_bf16_fp4(src, scf, 1)); break;
@@ -1962,9 +2077,10 @@ __device__ __forceinline__ void d5_tile(const Params& p, uint8_t* lds, int e, in
             }
           }
           if constexpr (HALF) {
-            if (pf && (i == 3 || i == 10)) issue_one(nxt_copy, o * 2 + (i == 3 ? 0 : 1));
+            const int j = o * 2 + (i == 3 ? 0 : 1);
+            if ((i == 3 || i == 10) && j < NCP) issue_one(nxt_copy, nso, j);
           } else {
-            if (pf && (i == 2 || i == 7 || i == 12)) issue_one(nxt_copy, o * 3 + (i == 2 ? 0 : i == 7 ? 1 : 2));
+            if (i == 2 || i == 7 || i == 12) issue_one(nxt_copy, nso, o * 3 + (i == 2 ? 0 : i == 7 ? 1 : 2));
           }
           __builtin_amdgcn_sched_barrier(0);
         }
@@ -1978,7 +2094,12 @@ __device__ __forceinline__ void d5_tile(const Params& p, uint8_t* lds, int e, in
           if (XC == 1 || (XC == 2 && odd)) {
 #pragma unroll
             for (int pg = 0; pg < PG; ++pg)
-              if (FULL || pg < pg_live) d5_cvt_exact(w[pg][0], w[pg][1], sc[pg], bf[nx][2 * pg], bf[nx][2 * pg + 1]);
+              if (FULL || pg < pg_live) {
+                uint32_t sb[8];
+#pragma unroll
+                for (int q = 0; q < 8; ++q) sb[q] = (sc[pg][q] >> 23) & 0xFFu;
+                d5_cvt_exact(w[pg][0], w[pg][1], sb, bf[nx][2 * pg], bf[nx][2 * pg + 1]);
+              }
           }
         }
       }
@@ -1989,46 +2110,22 @@ __device__ __forceinline__ void d5_tile(const Params& p, uint8_t* lds, int e, in
 #pragma unroll
     for (int tn = 0; tn < TN; ++tn) bf[1][tn] = zf;
     // a k-step's stage is complete once this wave's copies for it have landed
-    // (NCP newer ones outstanding (TS: 7), none for the last k-step)
-    if constexpr (HALF && TS) {
-      if (nk > 1)
-        AF3_ASM_WAIT_VM(7);
-      else
-        AF3_ASM_WAIT_VM(0);
-    } else if constexpr (HALF) {
-      if (nk > 1)
-        AF3_ASM_WAIT_VM(8);
-      else
-        AF3_ASM_WAIT_VM(0);
-    } else {
-      if (nk > 1)
-        AF3_ASM_WAIT_VM(12);
-      else
-        AF3_ASM_WAIT_VM(0);
-    }
+    // (the NCP newer ones may be outstanding)
+    auto wait_stage = [&] { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NCP) : "memory"); };
+    wait_stage();
     AF3_ASM_LDS_BARRIER();
-    kstep(0, true, nk > 2);
+    kstep(0, 0u, 2u * STAGE, true);
+    // the stage of k-step kt, and that of kt + 2 = kt - 1, carried as scalars
+    uint32_t so = STAGE, nso = 0u;
 #pragma nounroll
     for (int kt = 1; kt < nk; ++kt) {
-      if constexpr (HALF && TS) {
-        if (kt + 1 < nk)
-          AF3_ASM_WAIT_VM(7);
-        else
-          AF3_ASM_WAIT_VM(0);
-      } else if constexpr (HALF) {
-        if (kt + 1 < nk)
-          AF3_ASM_WAIT_VM(8);
-        else
-          AF3_ASM_WAIT_VM(0);
-      } else {
-        if (kt + 1 < nk)
-          AF3_ASM_WAIT_VM(12);
-        else
-          AF3_ASM_WAIT_VM(0);
-      }
+      wait_stage();
       AF3_ASM_LDS_BARRIER();
-      kstep(kt, false, kt + 2 < nk);
+      kstep(kt, so, nso, false);
+      nso = so;
+      so = so == 2u * STAGE ? 0u : so + STAGE;
     }
+    AF3_ASM_WAIT_VM(0);  // the repeated copies, before the LDS is reused
     // the last k-step's sub-step 3
 #pragma unroll
     for (int i = 0; i < TMW * TN; ++i) {
@@ -2153,6 +2250,37 @@ __global__ __launch_bounds__(256, 2) void gemm8_dgrad_kernel(Params p) {
     d5_tile<false, BXK, 1, 3, true, SA, TS>(p, lds, e, row_lo, nrows, n0, ncols);
   else
     d5_tile<false, BXK, 1, 0, true, SA, TS>(p, lds, e, row_lo, nrows, n0, ncols);
+}
+
+// The short-tile input gradient: RM x 256 items on the RM-row map (RM = 32 /
+// 64), gemm8's k-loop copying RM activation rows per k-step instead of 128, so
+// three (RM 64: two) blocks share a CU.  Each n-tile takes 128 bytes of every
+// packed weight row, so an expert's n-tiles run together on one XCD
+// (g4_work_item; dealt over the XCDs the launches were 15% slower).  Measured
+// (both launches of a backward): 301 tokens over 128 experts, rank 32, 420 -> 382
+// us, 1021 tokens 467 -> 449 (64 rows), 23 tokens over 32 experts 135 -> 124.
+template <int RM>
+constexpr int kG9DxLdsBytes = kD5Stages * (RM * 128 + 64 * 128 + 8 * 64 * 4);  // 42 / 54 KB
+static_assert(kG9DxLdsBytes<32> >= (32 + 256) * kBK * 2 && kG9DxLdsBytes<64> >= (64 + 256) * kBK * 2, "LoRA segment");
+static_assert(kG9DxLdsBytes<32> >= 32 * 512 + 2048 && kG9DxLdsBytes<64> >= 64 * 512 + 2048, "epilogue");
+
+template <int BXK, int RM, bool TS>
+__global__ __launch_bounds__(256, RM == 32 ? 3 : 2) void gemm9_dgrad_kernel(Params p) {
+  __shared__ __attribute__((aligned(16))) uint8_t lds[kG9DxLdsBytes<RM>];
+  int mt, nt;
+  if (!(p.tile_offs[p.E] < kG9SpreadTiles ? g9_work_item(p, mt, nt) : g4_work_item(p, mt, nt))) return;
+  const int32_t ent = p.tile_map[mt];
+  if (ent < 0) return;
+  const int e = ent & 0xFFFF, blk = ent >> 16;
+  const int row_lo = p.offs[e] + blk * RM;
+  const int nrows = min(RM, p.offs[e + 1] - row_lo);
+  if (nrows <= 0) return;
+  const int n0 = nt * 256;
+  const int ncols = min(256, p.N - n0);
+  if (RM == 64 && nrows <= 32)
+    d5_tile<false, BXK, 1, 1, true, true, TS, RM>(p, lds, e, row_lo, nrows, n0, ncols);
+  else
+    d5_tile<false, BXK, 1, 0, true, true, TS, RM>(p, lds, e, row_lo, nrows, n0, ncols);
 }
 
 // ---------------------------------------------------------------------------
@@ -2694,6 +2822,26 @@ static void launch_gemm7_fwd(int max_tiles, int N, hipStream_t stream, Params p)
   }
 }
 
+// short tiles: block_m 32 / 64 (moe_gemm_impl checks what they need)
+static void launch_gemm9(bool trans, int block_m, int max_tiles, int N, hipStream_t stream, Params p) {
+  p.n_nblk = (N + 255) / 256;
+  const int small = max_tiles < kG9SpreadTiles ? max_tiles : kG9SpreadTiles;
+  const unsigned spread = g9_grid(small, p.n_nblk, p.group_m), grouped = g4_grid(max_tiles, p.n_nblk, p.group_m);
+  dim3 grid(spread > grouped ? spread : grouped);
+#define AF3_G9(kern) hipLaunchKernelGGL(kern, grid, dim3(256), 0, stream, p)
+  if (!trans) {
+    if (block_m == 32) AF3_G9((gemm9_fwd_kernel<ROWS_BF16, 32>));
+    else AF3_G9((gemm9_fwd_kernel<ROWS_BF16, 64>));
+  } else if (p.s_tiled) {
+    if (block_m == 32) AF3_G9((gemm9_dgrad_kernel<COLS_BF16, 32, true>));
+    else AF3_G9((gemm9_dgrad_kernel<COLS_BF16, 64, true>));
+  } else {
+    if (block_m == 32) AF3_G9((gemm9_dgrad_kernel<COLS_BF16, 32, false>));
+    else AF3_G9((gemm9_dgrad_kernel<COLS_BF16, 64, false>));
+  }
+#undef AF3_G9
+}
+
 template <int BM, int BN, int WM, int WN>
 static void launch_gemm2(bool trans, int max_tiles, int N, hipStream_t stream, Params p) {
   p.n_nblk = (N + BN - 1) / BN;
@@ -2736,7 +2884,9 @@ static int moe_gemm_impl(const uint16_t* x, int64_t ldx, const int32_t* gather_i
   AF3_REQUIRE(lora_r == 0 || (lora_l && lora_b && ld_l % 8 == 0 && lora_r % 8 == 0 && al16(lora_l) && al16(lora_b)),
               "moe_gemm: LoRA operands must be 16-byte aligned, rank % 8 == 0");
   AF3_REQUIRE(al16(w_blocks), "moe_gemm: weight blocks must be 16-byte aligned");
-  AF3_REQUIRE(block_m == 128 || block_m == 256, "moe_gemm: block_m must be 128 or 256 (got %d)", block_m);
+  const bool short_tiles = block_m == 32 || block_m == 64;
+  AF3_REQUIRE(block_m == 128 || block_m == 256 || short_tiles, "moe_gemm: block_m must be 32, 64, 128 or 256 (got %d)",
+              block_m);
   Params p{};
   const int G_k = K / 32, G_n = N / 32;
   p.a = make_bf16(x, ldx, 0, gather_indx, gather_div);
@@ -2792,13 +2942,15 @@ static int moe_gemm_impl(const uint16_t* x, int64_t ldx, const int32_t* gather_i
   //   28: gemm8 input gradient (gemm5's k-loop on 128x256 items of the 128-row
   //       map, 4 waves of 128x64, two blocks per CU); default for trans_w 1
   //       with block_m 128
+  //   27 / 29: gemm9 forward / input gradient, gemm7's / gemm8's k-loop on 32 /
+  //       64 x 256 work items; default for block_m 32 and 64 (few rows per expert)
   //   23: gemm5 input gradient (packed weight rows read with transposing LDS
   //       loads, one three-stage ring for A, B and scales; 4 waves of 256x64);
   //       default for trans_w 1 with block_m 256
   //   4 / 2: gemm2, 256x256 / 128x256 tiles with the weight dequantised into
   //       LDS (general fallback for block_m 256 / 128)
   //   9: single-buffered 128x128 row tiles (any K % 32 == 0; used when K % 64 != 0)
-  //   tile_cfg / 100 = m-tiles per group of the 22 / 23 / 26 / 28 work order (default 4; 2 for 26 / 28)
+  //   tile_cfg / 100 = m-tiles per group of the 22 / 23 / 26 - 29 work order (default 4; 2 for 26 / 28)
   int cfg = tile_cfg % 100;
   const int group_m = tile_cfg / 100 > 0 ? tile_cfg / 100 : 4;
   if (cfg == 0) {
@@ -2809,11 +2961,25 @@ static int moe_gemm_impl(const uint16_t* x, int64_t ldx, const int32_t* gather_i
     const bool g4_dgrad = trans && block_m == 256 && K % kBK == 0 && N % 64 == 0 && al16(y) && ldy % 8 == 0;
     const bool g8_dgrad = trans && block_m == 128 && K % kBK == 0 && N % 64 == 0 && al16(y) && ldy % 8 == 0;
     cfg = g4_fwd ? 22 : g7_fwd ? 26 : g4_dgrad ? 23 : g8_dgrad ? 28 : (block_m == 256 ? 4 : 2);
+    if (short_tiles) cfg = trans ? 29 : 27;
   }
-  const bool bm_ok = (cfg == 4 || cfg == 22 || cfg == 23) ? block_m == 256 : block_m == 128;
+  if (cfg == 27 || cfg == 29) {
+    const bool ok = short_tiles && !a_fp8 && x_off32 && (int64_t)N * K / 2 < (1LL << 32) && al16(y) && ldy % 8 == 0 &&
+                    (trans ? cfg == 29 && K % kBK == 0 && N % 64 == 0
+                           : cfg == 27 && K % (kG9NB * kBK) == 0 && K / 32 <= kG7MaxG && N % 64 == 0 && al16(w_scales));
+    if (!ok) {
+      af3::set_error("moe_gemm: the short-tile kernels need block_m 32 or 64, x and an expert's weights within 4 GiB, "
+                     "N %% 64 == 0, K %% %d == 0 (trans_w 0, K <= %d) or K %% 64 == 0 (trans_w 1), 16-byte aligned y",
+                     kG9NB * kBK, kG7MaxG * 32);
+      return AF3_EUNSUPPORTED;
+    }
+  }
+  const bool bm_ok = (cfg == 4 || cfg == 22 || cfg == 23) ? block_m == 256
+                     : (cfg == 27 || cfg == 29)           ? short_tiles
+                                                          : block_m == 128;
   AF3_REQUIRE(bm_ok, "moe_gemm: tile_cfg %d does not match block_m %d", cfg, block_m);
   if (w_tiled) {  // only the two-blocks-per-CU forward reads the forward-tiled weights
-    if (a_fp8 || trans || cfg != 26 || K % kBK != 0) {
+    if (a_fp8 || trans || !(cfg == 26 || cfg == 27) || K % kBK != 0) {
       af3::set_error("moe_gemm: forward-tiled weights need the tile_cfg 26 forward (got cfg %d, trans_w %d)", cfg,
                      trans_w);
       return AF3_EUNSUPPORTED;
@@ -2821,7 +2987,7 @@ static int moe_gemm_impl(const uint16_t* x, int64_t ldx, const int32_t* gather_i
     p.b_tiled = 1;
   }
   if (s_tiled) {  // only the two-blocks-per-CU input gradient reads the tiled scales
-    if (a_fp8 || !trans || cfg != 28 || K % kBK != 0 || N % 64 != 0) {
+    if (a_fp8 || !trans || !(cfg == 28 || cfg == 29) || K % kBK != 0 || N % 64 != 0) {
       af3::set_error("moe_gemm: tiled input-gradient scales need tile_cfg 28 with trans_w 1 (got cfg %d, trans_w %d)",
                      cfg, trans_w);
       return AF3_EUNSUPPORTED;
@@ -2857,8 +3023,8 @@ static int moe_gemm_impl(const uint16_t* x, int64_t ldx, const int32_t* gather_i
   if (K % kBK != 0) cfg = 9;  // direct A loads need whole 64-deep k-steps (never with forward-tiled weights)
   if (epi != 0) {
     AF3_REQUIRE(glu && (epi == 1 || epi == 2), "moe_gemm: bad SwiGLU epilogue %d", epi);
-    const bool ok = epi == 1 ? (trans && (cfg == 23 || cfg == 28) && ld_glu % 8 == 0 && al16(glu) && ldy >= 2LL * N)
-                             : (!trans && (cfg == 22 || cfg == 26) && N % 2 == 0 && ld_glu % 4 == 0 &&
+    const bool ok = epi == 1 ? (trans && (cfg == 23 || cfg == 28 || cfg == 29) && ld_glu % 8 == 0 && al16(glu) && ldy >= 2LL * N)
+                             : (!trans && (cfg == 22 || cfg == 26 || cfg == 27) && N % 2 == 0 && ld_glu % 4 == 0 &&
                                 ((uintptr_t)glu & 7) == 0);
     if (!ok) {
       af3::set_error("moe_gemm: the fused SwiGLU epilogue %d is not available for tile_cfg %d / these operands", epi,
@@ -2868,8 +3034,8 @@ static int moe_gemm_impl(const uint16_t* x, int64_t ldx, const int32_t* gather_i
   }
   if (a_row_scale) {
     AF3_REQUIRE(lora_r == 0, "moe_gemm: a row scale cannot be combined with the LoRA extension segment");
-    if (!(cfg == 22 || cfg == 23 || cfg == 26 || cfg == 28)) {
-      af3::set_error("moe_gemm: the A row scale needs tile_cfg 22, 23, 26 or 28 (got %d)", cfg);
+    if (!(cfg == 22 || cfg == 23 || (cfg >= 26 && cfg <= 29))) {
+      af3::set_error("moe_gemm: the A row scale needs tile_cfg 22, 23 or 26 - 29 (got %d)", cfg);
       return AF3_EUNSUPPORTED;
     }
   }
@@ -2894,6 +3060,11 @@ static int moe_gemm_impl(const uint16_t* x, int64_t ldx, const int32_t* gather_i
                       ldy % 8 == 0,
                   "moe_gemm: tile_cfg 26 needs trans_w 0, block_m 128, K %% 64 == 0, K <= %d, 16-byte aligned", kG7MaxG * 32);
       launch_gemm7_fwd(max_tiles, N, stream, p);
+      break;
+    case 27:
+    case 29:
+      p.group_m = tile_cfg / 100 > 0 ? tile_cfg / 100 : 2;
+      launch_gemm9(trans, block_m, max_tiles, N, stream, p);
       break;
     case 28:
       p.group_m = tile_cfg / 100 > 0 ? tile_cfg / 100 : 2;

@@ -147,16 +147,19 @@ int af3_tile_order(const int32_t* hist, int n_expts_tot, int block_m, const int3
  *   Y = bf16((acc + bias[e][n]) * gammas[r])   (bias fp32 [E][N], gammas bf16 or fp32)
  * a(r) = gather_indx ? gather_indx[r] / gather_div : r; rows r of expert e
  * are [token_offs[e], token_offs[e+1]); block_pid_map / tile_offs are the
- * af3_expt_data map and token_offs_pad for BM = block_m (128 or 256); the
+ * af3_expt_data map and token_offs_pad for BM = block_m (32, 64, 128 or 256); the
  * number of valid m-tiles is read from tile_offs[n_expts] on the device.
  * tile_cfg picks the block tile; 0 = the default for block_m and trans_w:
  * block_m 128 -> 26 (forward, 128 x 256 work items, two blocks per CU) and
- * 28 (input gradient, same shape); block_m 256 -> 22 / 23 (256 x 256); the
+ * 28 (input gradient, same shape); block_m 32 / 64 -> 27 / 29, the same k-loops
+ * on 32 / 64 x 256 items for few rows per expert (AF3_EUNSUPPORTED, nothing
+ * launched, unless AF3_X_OFFSETS_32 is set, N % 64 == 0 and K % 320 == 0 (27; K
+ * <= 3072) or K % 64 == 0 (29)); block_m 256 -> 22 / 23 (256 x 256); the
  * general fallbacks 4 / 2 / 9 where a default's alignment or K % 64 == 0
  * requirement fails.  tile_cfg / 100 = m-tiles per work group of the
  * 22 / 23 / 26 / 28 order (default 4; 2 for 26 / 28).  tile_cfg |
  * AF3_W_FWD_TILED: w_blocks is the af3_mxfp4_tile_fwd copy of the weights
- * (trans_w 0, the tile_cfg 26 forward only; AF3_EUNSUPPORTED, nothing
+ * (trans_w 0, the tile_cfg 26 / 27 forward only; AF3_EUNSUPPORTED, nothing
  * launched, when another kernel is selected: the caller then passes the
  * row-major blocks).  tile_cfg | AF3_X_OFFSETS_32: the caller vouches that
  * every row of x the call reads lies within 4 GiB of x (a(r) * ldx * 2 + K * 2
@@ -216,7 +219,7 @@ int af3_mxfp4_tile_dx_scales(const uint8_t* scales, int64_t n_mats, int K, int N
  * 516-525, 432-439: epi 2, trans_w 0, y <- the bf16 pre-activation [rows][N]
  * and glu <- its SwiGLU [rows][N/2]).  Results equal the unfused sequence bit
  * for bit.  Returns AF3_EUNSUPPORTED (-2) when the selected tile configuration
- * has no fused epilogue (epi 2: tile_cfg 22 / 26, epi 1: 23 / 28); the caller
+ * has no fused epilogue (epi 2: tile_cfg 22 / 26 / 27, epi 1: 23 / 28 / 29); the caller
  * then runs the unfused pair. */
 int af3_moe_gemm_swiglu(const uint16_t* x, int64_t ldx, const int32_t* gather_indx, int gather_div,
                         const uint8_t* w_blocks, const uint8_t* w_scales, int trans_w, const float* bias,
@@ -233,7 +236,7 @@ int af3_moe_gemm_swiglu(const uint16_t* x, int64_t ldx, const int32_t* gather_in
  * scale_mode="per_token")) in the fp8 mode, quantization.py:338-356 (forward)
  * and 382-408 (dX), fed with the E4M3 codes' values as bf16.  Returns
  * AF3_EUNSUPPORTED (-2) when the selected tile configuration has no scaled
- * epilogue (only tile_cfg 22, 23, 26 and 28 have one). */
+ * epilogue (only tile_cfg 22, 23 and 26 - 29 have one). */
 int af3_moe_gemm_rowscale(const uint16_t* x, int64_t ldx, const int32_t* gather_indx, int gather_div,
                           const uint8_t* w_blocks, const uint8_t* w_scales, int trans_w, const float* bias,
                           const void* gammas, int gammas_f32, const int32_t* token_offs, const int32_t* block_pid_map,

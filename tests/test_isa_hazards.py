@@ -40,6 +40,16 @@ def test_forward_weight_loads_have_no_register_hazard(moe_gemm_asm, symbol):
     assert not bad, bad[:5]
 
 
+@pytest.mark.timeout(600)
+@pytest.mark.parametrize("rows", [32, 64])
+def test_short_tile_weight_loads_have_no_register_hazard(moe_gemm_asm, rows):
+    """The short-tile forward: five weight-register buffers, four k-steps in flight."""
+    n, bad = H.violations(H.function_body(moe_gemm_asm,
+                                          f"_ZN12_GLOBAL__N_116gemm9_fwd_kernelILi0ELi{rows}EEEvNS_6ParamsE"))
+    assert n >= 18, "expected the prologue's and the k-loop's inline-assembly weight loads"
+    assert not bad, bad[:5]
+
+
 def test_checker_finds_planted_hazards():
     base = ["s_waitcnt vmcnt(0)", ";;#ASMSTART", "global_load_dwordx4 v[8:11], v[2:3], off", ";;#ASMEND"]
     ok = base + ["global_load_lds_dwordx4 v[4:5], off", "s_waitcnt vmcnt(1)", "v_mov_b32_e32 v0, v8", "s_endpgm"]
