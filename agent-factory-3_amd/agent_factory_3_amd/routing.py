@@ -30,7 +30,8 @@ BLOCK_MS = (128, 256, 512)
 GEMM_ORDER_BMS = (128,)  # tile sizes whose full-first work order is made with the routing (the
 # default GEMMs and the LoRA row tiles); other sizes get theirs on first use (gemm_order_for)
 SHORT_BLOCK_MS = (32, 64)  # tile sizes of the short-tile GEMMs, mapped where the rows are few per expert
-SHORT_ROWS_PER_EXPERT = 64  # (routed rows <= this many per expert)
+SHORT_ROWS_PER_EXPERT = 64  # (routed rows <= this many per expert, or at most SHORT_TILES 32-row tiles)
+SHORT_TILES = 512
 PLAN_MAX_E = 1024  # experts of af3_routing_plan (routing and tile metadata in one call)
 
 
@@ -188,7 +189,7 @@ def _routing_plan(lg: torch.Tensor, K: int, ei: torch.Tensor | None, ld: int):
     T, E = lg.shape
     R = T * K
     dev = lg.device
-    bms = SHORT_BLOCK_MS + BLOCK_MS if R <= SHORT_ROWS_PER_EXPERT * E else BLOCK_MS
+    bms = SHORT_BLOCK_MS + BLOCK_MS if R <= SHORT_ROWS_PER_EXPERT * E or max_tiles(R, E, 32) <= SHORT_TILES else BLOCK_MS
     nb = len(bms)
     tiles = [max_tiles(R, E, bm) for bm in bms]
     mt = max(tiles)

@@ -23,7 +23,7 @@ int check_launch(const char* what);
 // not covered (the entry points then use the general kernels)
 int lora_rows_fast(const uint16_t* x, int64_t ldx, const int32_t* gather, int gdiv, const uint16_t* wl, int trans_b,
                    float scale, const int32_t* token_offs, const int32_t* block_pid_map, int max_tiles, int n_out,
-                   int K, uint16_t* out, int64_t ld_out, hipStream_t stream);
+                   int K, uint16_t* out, int64_t ld_out, int rows32, hipStream_t stream);
 int lora_wgrad_fast(const uint16_t* big, int64_t ld_big, const int32_t* big_gather, int big_div,
                     const uint16_t* small, int64_t ld_small, const uint16_t* rowscale, int small_is_a, int W, int r,
                     float scale, const int32_t* token_offs, const int32_t* chunk_map, const int32_t* chunk_offs,
@@ -41,6 +41,10 @@ int lora_wgrad_fast(const uint16_t* big, int64_t ld_big, const int32_t* big_gath
 // within 4 GiB of x (row * ldx * 2 + K * 2 <= 2^32)
 #ifndef AF3_X_OFFSETS_32
 #define AF3_X_OFFSETS_32 0x20000
+#endif
+// OR-ed into af3_lora_rows' trans_b: block_pid_map is the map of 32-row tiles
+#ifndef AF3_LORA_ROWS_32
+#define AF3_LORA_ROWS_32 0x100
 #endif
 // OR-ed into af3_moe_gemm's tile_cfg: w_scales is the af3_mxfp4_tile_dx_scales copy
 #ifndef AF3_S_DX_TILED

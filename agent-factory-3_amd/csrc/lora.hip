@@ -95,6 +95,12 @@ __device__ __forceinline__ int l_swz(int row) { return (row ^ (row >> 3)) & 7; }
 // TRANS) go global->LDS through a 2-stage ring, one k-step ahead: 40 KB of
 // LDS, so four blocks fit a CU and the ~640 blocks of a 65,536-row layer run
 // in one round instead of 1.25 rounds of two blocks per CU.
+// With few rows per expert there is about one block per CU, and one k-step's
+// load latency times K / 64 steps is all the launch costs (32-37 us from 23 to
+// 1021 tokens): RT = 32 takes the 32-row map, one wave computing, through an
+// 8-stage ring with seven k-steps in flight.  Measured, the two launches
+// of a forward: 23 tokens over 32 experts 72 -> 35 us, 1021 tokens over 128 83
+// -> 48, 2000 tokens over 32 (250 rows per expert) 82 -> 49.
 // ---------------------------------------------------------------------------
 struct LrParams {
   const uint16_t* x;
@@ -111,20 +117,20 @@ struct LrParams {
   int64_t ld_out;
 };
 
-constexpr int kLrA = 128 * 64 * 2;  // A bytes per stage
 constexpr int kLrB = 64 * 64;       // B bytes per stage (<= 32 x 64 bf16)
-constexpr int kLrStage = kLrA + kLrB;
 
-constexpr int kLrStages = 2;
-
-template <bool TRANS, int SR>
+// RT rows per tile (128 or 32), ST ring stages
+template <bool TRANS, int SR, int RT, int ST>
 __global__ __launch_bounds__(256) void lrows_kernel(LrParams p) {
-  __shared__ __attribute__((aligned(16))) uint8_t lds[kLrStages * kLrStage];
+  constexpr int kLrA = RT * 64 * 2;  // A bytes per stage
+  constexpr int kLrStage = kLrA + kLrB;
+  constexpr int AI = RT / 32;        // A copies per wave and k-step (8 rows each)
+  __shared__ __attribute__((aligned(16))) uint8_t lds[ST * kLrStage];
   const int32_t ent = p.tile_map[blockIdx.x];
   if (ent < 0) return;
   const int e = ent & 0xFFFF, blk = ent >> 16;
-  const int row_lo = p.offs[e] + blk * 128;
-  const int nrows = min(128, p.offs[e + 1] - row_lo);
+  const int row_lo = p.offs[e] + blk * RT;
+  const int nrows = min(RT, p.offs[e + 1] - row_lo);
   if (nrows <= 0) return;
   const int nk = p.K / 64;
   const int lane = threadIdx.x & 63;
@@ -133,11 +139,10 @@ __global__ __launch_bounds__(256) void lrows_kernel(LrParams p) {
   constexpr int NB = TRANS ? (64 * SR) / 1024 : 4;  // B copies per stage (block)
   const bool has_b = wave < NB;
 
-  // A: 4 copies per wave (8 rows each)
-  const uint16_t* arow[4];
+  const uint16_t* arow[AI];
 #pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    const int row = (wave * 4 + i) * 8 + (lane >> 3);
+  for (int i = 0; i < AI; ++i) {
+    const int row = (wave * AI + i) * 8 + (lane >> 3);
     int64_t src = row_lo + (row < nrows ? row : 0);
     if (p.gather) src = p.gather[src] / p.gdiv;
     arow[i] = p.x + src * p.ldx + (((lane & 7) ^ l_swz(row)) << 3);
@@ -157,24 +162,34 @@ __global__ __launch_bounds__(256) void lrows_kernel(LrParams p) {
   }
   const int64_t bstep = TRANS ? (int64_t)64 * p.r * 2 : 128;
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane(l_lds_addr(lds));
+  // (ST > 2: the k-steps past the end copy the last one again, into a stage no wave reads again)
   auto issue = [&](int kt) {
-    const uint32_t st = lds0 + (uint32_t)((kt % kLrStages) * kLrStage);
+    const uint32_t st = lds0 + (uint32_t)((kt % ST) * kLrStage);
+    const int ks = ST > 2 ? min(kt, nk - 1) : kt;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) l_dma16(arow[i] + kt * 64, st + (uint32_t)((wave * 4 + i) * 1024));
-    if (has_b) l_dma16(bsrc + kt * bstep, st + (uint32_t)(kLrA + wave * 1024));
+    for (int i = 0; i < AI; ++i) l_dma16(arow[i] + ks * 64, st + (uint32_t)((wave * AI + i) * 1024));
+    if (has_b) l_dma16(bsrc + ks * bstep, st + (uint32_t)(kLrA + wave * 1024));
   };
   af3_f32x16 acc;
 #pragma unroll
   for (int q = 0; q < 16; ++q) acc[q] = 0.f;
 
-  issue(0);
+#pragma unroll
+  for (int k = 0; k < ST - 1; ++k) issue(k);
   for (int kt = 0; kt < nk; ++kt) {
-    // this k-step's copies are the only ones in flight; the barrier also orders
-    // every wave's reads of the other stage (k-step kt - 1) before its refill
-    L_WAIT_VM(0);
+    // this k-step's copies have landed (ST 2: the only ones in flight; else the
+    // ST - 2 newer k-steps' may be outstanding); the barrier also orders every
+    // wave's reads of stage kt - 1 before its refill
+    if constexpr (ST == 2) {
+      L_WAIT_VM(0);
+    } else {
+      static_assert((ST - 2) * (AI + 1) <= 31, "wait counts");
+      l_wait_vm((ST - 2) * (AI + (has_b ? 1 : 0)));
+    }
     L_BARRIER();
-    if (kt + 1 < nk) issue(kt + 1);
-    const uint8_t* as = lds + (kt % kLrStages) * kLrStage;
+    if (ST > 2 || kt + 1 < nk) issue(kt + ST - 1);
+    if (wave * 32 >= RT) continue;  // a wave that only copies
+    const uint8_t* as = lds + (kt % ST) * kLrStage;
     const uint8_t* bs = as + kLrA;
 #pragma unroll
     for (int s = 0; s < 4; ++s) {
@@ -192,8 +207,9 @@ __global__ __launch_bounds__(256) void lrows_kernel(LrParams p) {
       acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, acc, 0, 0, 0);
     }
   }
+  if constexpr (ST > 2) L_WAIT_VM(0);  // the repeated copies, before the LDS is given back
   const int j = lr;
-  if (j < p.r) {
+  if (j < p.r && wave * 32 < RT) {
 #pragma unroll
     for (int q = 0; q < 16; ++q) {
       const int row = wave * 32 + (q >> 2) * 8 + lh * 4 + (q & 3);
@@ -749,7 +765,7 @@ namespace af3 {
 
 int lora_rows_fast(const uint16_t* x, int64_t ldx, const int32_t* gather, int gdiv, const uint16_t* wl, int trans_b,
                    float scale, const int32_t* token_offs, const int32_t* block_pid_map, int max_tiles, int n_out,
-                   int K, uint16_t* out, int64_t ld_out, hipStream_t stream) {
+                   int K, uint16_t* out, int64_t ld_out, int rows32, hipStream_t stream) {
   if (!(n_out == 16 || n_out == 32) || K % 64 != 0 || ldx % 8 != 0 || !l_al16(x) || !l_al16(wl)) return AF3_EUNSUPPORTED;
   LrParams p{};
   p.x = x;
@@ -766,12 +782,20 @@ int lora_rows_fast(const uint16_t* x, int64_t ldx, const int32_t* gather, int gd
   p.out = out;
   p.ld_out = ld_out;
   const dim3 grid(max_tiles), block(256);
+#define AF3_LR(tr, sr)                                                                          \
+  do {                                                                                           \
+    if (rows32)                                                                                  \
+      hipLaunchKernelGGL((lrows_kernel<tr, sr, 32, 8>), grid, block, 0, stream, p);              \
+    else                                                                                         \
+      hipLaunchKernelGGL((lrows_kernel<tr, sr, 128, 2>), grid, block, 0, stream, p);             \
+  } while (0)
   if (trans_b == 0)
-    hipLaunchKernelGGL((lrows_kernel<false, 64>), grid, block, 0, stream, p);
+    AF3_LR(false, 64);
   else if (n_out == 32)
-    hipLaunchKernelGGL((lrows_kernel<true, 64>), grid, block, 0, stream, p);
+    AF3_LR(true, 64);
   else
-    hipLaunchKernelGGL((lrows_kernel<true, 32>), grid, block, 0, stream, p);
+    AF3_LR(true, 32);
+#undef AF3_LR
   return check_launch("lora_rows");
 }
 

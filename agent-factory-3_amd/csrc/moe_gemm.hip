@@ -3166,12 +3166,18 @@ extern "C" int af3_lora_rows(const uint16_t* x, int64_t ldx, const int32_t* gath
   hipStream_t stream = (hipStream_t)stream_;
   AF3_REQUIRE(n_out > 0 && n_out <= 64 && K > 0, "lora_rows: bad sizes n_out=%d K=%d", n_out, K);
   if (max_tiles == 0) return 0;
+  const int rows32 = (trans_b & AF3_LORA_ROWS_32) != 0;  // block_pid_map is the 32-row map
+  trans_b &= ~AF3_LORA_ROWS_32;
   AF3_REQUIRE(K % 8 == 0 && n_out % 8 == 0 && ldx % 8 == 0 && al16(x) && al16(wl),
               "lora_rows: operands must be 16-byte aligned with sizes % 8 == 0");
   {
     const int rc = af3::lora_rows_fast(x, ldx, gather_indx, gather_div, wl, trans_b, scale, token_offs, block_pid_map,
-                                       max_tiles, n_out, K, out, ld_out, stream);
+                                       max_tiles, n_out, K, out, ld_out, rows32, stream);
     if (rc != AF3_EUNSUPPORTED) return rc;
+  }
+  if (rows32) {
+    af3::set_error("lora_rows: the 32-row map needs rank 16 or 32, K %% 64 == 0 and 16-byte aligned operands");
+    return AF3_EUNSUPPORTED;
   }
   Params p{};
   p.a = make_bf16(x, ldx, 0, gather_indx, gather_div);

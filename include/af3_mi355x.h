@@ -293,6 +293,12 @@ int af3_moe_combine(const uint16_t* rows, int64_t ld_rows, const int32_t* src_in
  * no expert LoRA; convention dW = scale * B @ A of model_trainer.py:665,711):
  *   trans_b 0: out[r][j] = scale * sum_k X[a(r)][k] Wl[e][j][k]
  *   trans_b 1: out[r][j] = scale * sum_k X[a(r)][k] Wl[e][k][j]        */
+/* trans_b | AF3_LORA_ROWS_32: block_pid_map is the map of 32-row tiles (few rows
+ * per expert; n_out 16 or 32 and K % 64 == 0, else AF3_EUNSUPPORTED with nothing
+ * launched) instead of the 128-row one. */
+#ifndef AF3_LORA_ROWS_32
+#define AF3_LORA_ROWS_32 0x100
+#endif
 int af3_lora_rows(const uint16_t* x, int64_t ldx, const int32_t* gather_indx, int gather_div, const uint16_t* wl,
                   int trans_b, float scale, const int32_t* token_offs, const int32_t* block_pid_map, int max_tiles,
                   int n_expts, int n_out, int K, uint16_t* out, int64_t ld_out, void* stream);

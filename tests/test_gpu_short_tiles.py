@@ -120,5 +120,25 @@ def test_map_choice(dev):
     assert Q._short_block_m(ed, 400, 32, 96, 2880, True, True) == 0          # N % 64
     assert Q._short_block_m(ed, 400, 32, 5760, 2880, False, False) == 0      # 64-bit offsets
     assert Q._short_block_m(ed, 1 << 20, 32, 5760, 2880, False, True) == 0
-    big = R.routing(torch.randn(2000, 16, device=dev).to(torch.bfloat16), 4)[0].expt_data
+    big = R.routing(torch.randn(8000, 16, device=dev).to(torch.bfloat16), 4)[0].expt_data     # 2000 rows per expert
     assert 32 not in big.block_pid_map and Q._short_block_m(big, 100, 16, 5760, 2880, False, True) == 0
+
+
+@pytest.mark.parametrize("r", [16, 32])
+@pytest.mark.parametrize("trans_b,K", [(0, 64), (0, 576), (0, 2880), (1, 128), (1, 1472)])
+def test_lora_rows_32_row_map(dev, monkeypatch, r, trans_b, K):
+    """The 32-row LoRA row product: bit-equal to the 128-row one on every tile edge (fewer k-steps than
+    ring stages included), with and without a gather."""
+    g = torch.Generator().manual_seed(K + r)
+    E = len(HIST)
+    rd, n = _routing(dev, HIST)
+    ed = rd.expt_data
+    x = torch.randn(n, K + 8, generator=g).to(torch.bfloat16).to(dev)[:, :K]
+    wl = torch.randn(*((E, K, r) if trans_b else (E, r, K)), generator=g).to(torch.bfloat16).to(dev)
+    idx = torch.randint(0, 2 * n, (n,), generator=g, dtype=torch.int32).to(dev)
+    for gather, k in ((None, 1), (idx, 2)):
+        out = []
+        for lim in (0, 1 << 20):
+            monkeypatch.setattr(Q, "LORA_SHORT_TILES", lim)
+            out.append(Q._lora_rows(x, gather, k, wl, trans_b, 0.5, ed, r, K))
+        assert torch.equal(out[0], out[1])
