@@ -44,7 +44,7 @@ fallback.
 from __future__ import annotations
 
 import math
-from contextlib import contextmanager
+from contextlib import nullcontext
 
 import torch
 from torch import nn
@@ -104,17 +104,19 @@ FP4_VALUES = [
 ]
 
 
-@contextmanager
+_HERE = nullcontext()
+
+
 def on_device(dev):
+    """Context with ``dev`` (a device, its name, or a tensor on it) as the current
+    GPU; nothing to do, and nothing done, when it already is."""
     if isinstance(dev, torch.Tensor):
         dev = dev.device
     elif isinstance(dev, str):
         dev = torch.device(dev)
-    if getattr(dev, "type", None) == "cuda":
-        with torch.cuda.device(dev):
-            yield
-            return
-    yield
+    if getattr(dev, "type", None) != "cuda" or dev.index is None or dev.index == torch.cuda.current_device():
+        return _HERE
+    return torch.cuda.device(dev)
 
 
 # ---------------------------------------------------------------------------
@@ -175,8 +177,9 @@ def _pack_uint8_as_bf16(tensor):
 
 def _unpack_bf16_as_uint8(packed, shape):
     """View bf16-packed bytes as a uint8 tensor of ``shape`` (no copy)."""
+    flat = (packed if packed.dim() == 1 else packed.reshape(-1)).view(torch.uint8)
     numel = math.prod(shape)
-    return packed.reshape(-1).view(torch.uint8)[:numel].reshape(shape)
+    return (flat if flat.shape[0] == numel else flat[:numel]).view(shape)
 
 
 def _store_mxfp4_weights(blocks, scales, module, proj, target_device):
@@ -555,7 +558,7 @@ class DequantMoEMatmul(torch.autograd.Function):
                 out = y if fwd_scatter_indx is None else moe_combine(y, fwd_scatter_indx, k)
             else:  # matmul_ogs(x, (blocks, scales), ...) with the module's forward-tiled weights
                 y = moe_rows(x, blocks, scales, bias, routing_data, fwd_gather_indx, fwd_gammas, False,
-                             w_tiled=_fwd_weights(experts_module, proj_name))
+                             w_tiled=_fwd_weights(experts_module, proj_name, blocks))
                 k = routing_data.n_expts_act if routing_data is not None else 1
                 out = y if fwd_scatter_indx is None else moe_combine(y, fwd_scatter_indx, k)
         ctx.experts_module = experts_module
@@ -598,7 +601,7 @@ class DequantMoEMatmul(torch.autograd.Function):
                                         ctx.bwd_scatter_indx, ctx.bwd_gammas, trans_w=True, a_row_scale=gs)
             else:  # matmul_ogs(g, (blocks, scales), ..., trans_w=True) with the module's tiled scales
                 y = moe_rows(g, blocks, scales, None, ctx.routing_data, ctx.bwd_gather_indx, ctx.bwd_gammas, True,
-                             s_tiled=_dx_scales(ctx.experts_module, ctx.proj_name))
+                             s_tiled=_dx_scales(ctx.experts_module, ctx.proj_name, scales))
                 k = ctx.routing_data.n_expts_act if ctx.routing_data is not None else 1
                 grad_x = y if ctx.bwd_scatter_indx is None else moe_combine(y, ctx.bwd_scatter_indx, k)
             d_gam = None
@@ -742,7 +745,7 @@ class LoraDequantMoEMatmul(torch.autograd.Function):
         with on_device(dev):
             L = _lora_rows(xg, g, k_act, A, 0, scaling, ed, r, K)
             y = moe_rows(xg, blocks, scales, bias, routing_data, fwd_gather_indx, fwd_gammas, False, L, B,
-                         w_tiled=_fwd_weights(experts_module, proj_name))
+                         w_tiled=_fwd_weights(experts_module, proj_name, blocks))
             if fwd_scatter_indx is not None:
                 y = moe_combine(y, fwd_scatter_indx, k_act)
         ctx.save_for_backward(xg, A, B, L)
@@ -779,7 +782,7 @@ class LoraDequantMoEMatmul(torch.autograd.Function):
         with on_device(dY.device):
             u, dB = _lora_u_and_dB(dY, bg, k_act if bg is not None else 1, gam, L, B, ctx.scaling, ed, E, N)
             dx = moe_rows(dY, blocks, scales, None, ctx.routing_data, ctx.bwd_gather_indx, gam, True, u, A,
-                          s_tiled=_dx_scales(ctx.experts_module, ctx.proj_name))
+                          s_tiled=_dx_scales(ctx.experts_module, ctx.proj_name, scales))
             if ctx.bwd_scatter_indx is not None:
                 dx = moe_combine(dx, ctx.bwd_scatter_indx, k_act)
             dA = _lora_wgrad(u, None, 1, gam, xg, ctx.fwd_gather, k_act if ctx.fwd_gather is not None else 1,
@@ -813,20 +816,20 @@ def _weights_of(ctx):
     return ctx.weights
 
 
-def _fwd_weights(experts_module, proj_name):
+def _fwd_weights(experts_module, proj_name, blocks):
     """The module's forward-tiled copy of ``proj_name``'s packed weights (None
     without a module or with FWD_TILED_WEIGHTS off)."""
     if experts_module is None or not FWD_TILED_WEIGHTS:
         return None
-    return experts_module._fwd_tiled(proj_name)
+    return experts_module._fwd_tiled(proj_name, blocks)
 
 
-def _dx_scales(experts_module, proj_name):
+def _dx_scales(experts_module, proj_name, scales):
     """The module's tiled copy of ``proj_name``'s scales for the input
     gradient (None without a module or with DX_TILED_SCALES off)."""
     if experts_module is None or not DX_TILED_SCALES:
         return None
-    return experts_module._dx_tiled_scales(proj_name)
+    return experts_module._dx_tiled_scales(proj_name, scales)
 
 
 def _bf16c(t):
@@ -853,7 +856,7 @@ class _GateUpSwiGLU(torch.autograd.Function):
         with on_device(dev):
             if A is not None:
                 L = _lora_rows(xg, g, k_act, A, 0, scaling, ed, A.shape[1], K)
-            wf = _fwd_weights(experts_module, proj_name)
+            wf = _fwd_weights(experts_module, proj_name, blocks)
             res = moe_rows(xg, blocks, scales, bias, routing_data, gather_indx, None, False, L, B,
                            swiglu=("fwd", alpha, limit), w_tiled=wf)
             if res is None:
@@ -892,7 +895,7 @@ class _GateUpSwiGLU(torch.autograd.Function):
                 u, dB = _lora_u_and_dB(dGU, None, 1, None, L, B, ctx.scaling, ed, E, N)
                 dB = dB.to(ctx.lora_dtypes[1])
             dx = moe_rows(dGU, blocks, scales, None, ctx.routing_data, None, None, True, u, A,
-                          s_tiled=_dx_scales(ctx.experts_module, ctx.proj_name))
+                          s_tiled=_dx_scales(ctx.experts_module, ctx.proj_name, scales))
             if ctx.scatter_indx is not None:
                 dx = moe_combine(dx, ctx.scatter_indx, k_act)
             if A is not None:
@@ -922,7 +925,7 @@ class _SwiGLUDown(torch.autograd.Function):
             if A is not None:
                 L = _lora_rows(act, None, 1, A, 0, scaling, ed, A.shape[1], K)
             y = moe_rows(act, blocks, scales, bias, routing_data, None, gammas, False, L, B,
-                         w_tiled=_fwd_weights(experts_module, proj_name))
+                         w_tiled=_fwd_weights(experts_module, proj_name, blocks))
             if scatter_indx is not None:
                 y = moe_combine(y, scatter_indx, k_act)
         # gate_up (the SwiGLU's input, the same bytes as the reference's saved
@@ -964,10 +967,10 @@ class _SwiGLUDown(torch.autograd.Function):
             if FUSED_SWIGLU_BWD and not want_gam:
                 dgu = moe_rows(dY, blocks, scales, None, ctx.routing_data, ctx.bwd_gather_indx, gam, True, u, A,
                                swiglu=("bwd", gate_up, ctx.alpha, ctx.limit),
-                               s_tiled=_dx_scales(ctx.experts_module, ctx.proj_name))
+                               s_tiled=_dx_scales(ctx.experts_module, ctx.proj_name, scales))
             if dgu is None:
                 d_act = moe_rows(dY, blocks, scales, None, ctx.routing_data, ctx.bwd_gather_indx, gam, True, u, A,
-                                 s_tiled=_dx_scales(ctx.experts_module, ctx.proj_name))
+                                 s_tiled=_dx_scales(ctx.experts_module, ctx.proj_name, scales))
                 if want_gam:
                     d_gam = _gamma_grad(d_act, act, dY, ctx.bwd_gather_indx, k_act, ctx.gamma_bias,
                                         ctx.routing_data, ctx.gammas)
@@ -1041,11 +1044,13 @@ class Mxfp4Bf16DequantGptOssExperts(nn.Module):
             hit = cache[proj] = (b, (b.data_ptr(), b._version), b.detach().float())
         return hit[2]
 
-    def _fwd_tiled(self, proj):
+    def _fwd_tiled(self, proj, blocks=None):
         """The forward-tiled copy of the projection's packed weights
         (``mxfp4_tile_fwd``), made once per weight storage and version (the
-        expert weights are frozen); None where the forward cannot read one."""
-        blocks, _ = self._get_uint8_weights(proj)
+        expert weights are frozen); None where the forward cannot read one.
+        ``blocks``: the projection's current uint8 blocks, where the caller has them."""
+        if blocks is None:
+            blocks, _ = self._get_uint8_weights(proj)
         if not blocks.is_cuda or blocks.dim() != 4 or blocks.shape[1] % 32 or blocks.shape[2] % 2:
             return None
         src = getattr(self, f"{proj}_blocks", None)
@@ -1062,11 +1067,13 @@ class Mxfp4Bf16DequantGptOssExperts(nn.Module):
                 hit = cache[proj] = (src, key, mxfp4_tile_fwd(blocks))
         return hit[2]
 
-    def _dx_tiled_scales(self, proj):
+    def _dx_tiled_scales(self, proj, scales=None):
         """The input gradient's tiled copy of the projection's scales
         (``mxfp4_tile_dx_scales``), made once per scale storage and version;
-        None where the input-gradient kernel cannot read one."""
-        _, scales = self._get_uint8_weights(proj)
+        None where the input-gradient kernel cannot read one.  ``scales``: the
+        projection's current uint8 scales, where the caller has them."""
+        if scales is None:
+            _, scales = self._get_uint8_weights(proj)
         if not scales.is_cuda or scales.dim() != 3 or scales.shape[1] % 64:
             return None
         src = getattr(self, f"{proj}_scales", None)
