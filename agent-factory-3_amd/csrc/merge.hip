@@ -13,14 +13,17 @@
 // 1 = [E][K][N] (transformers' GptOssExperts parameter, modeling_gpt_oss.py:75-77,
 // the layout a bf16 gpt-oss checkpoint holds).
 //
-// A tile = 64(n) x 64(k) of one expert; persistent blocks of 4 waves walk the tiles.  The rank-r delta
-// runs on v_mfma_f32_32x32x16_bf16 (products of bf16 are exact in fp32), each
-// wave one 32x32 sub-tile (A's k-slice staged in LDS with 16-byte loads), the
-// result staged in LDS as fp32.  Then each thread
-// dequantises a quarter MXFP4 block (8 values) of two rows, adds the delta and
-// writes 16 B of bf16 per row: straight to HBM for layout 0, through an LDS
-// transpose for layout 1 (64-column runs of 128 B, whole lines per store).  HBM-bound: per output element 2 B written
-// and 17/32 B of packed weight read; the adapters are re-read from L2.
+// Ranks above 64 take the general kernel: a tile = 64(n) x 64(k) of one expert,
+// persistent blocks of 4 waves walk the tiles.  The rank-r delta runs on
+// v_mfma_f32_32x32x16_bf16 (products of bf16 are exact in fp32), each wave one
+// 32x32 sub-tile (A's k-slice staged in LDS with 16-byte loads), the result
+// staged in LDS as fp32.  Then each thread dequantises a quarter MXFP4 block (8
+// values) of two rows, adds the delta and writes 16 B of bf16 per row: straight to
+// HBM for layout 0, through an LDS transpose for layout 1 (64-column runs of 128
+// B, whole lines per store).  HBM-bound: per output element 2 B written and 17/32
+// B of packed weight read; the adapters are re-read from L2.
+#include <type_traits>
+
 #include "af3_common.h"
 
 namespace {
@@ -196,186 +199,196 @@ __global__ __launch_bounds__(256, 6) void lora_merge_generic_kernel(const uint8_
   }
 }
 
-// The merge for r <= 64.  A block owns one (expert, 64-column k-tile, run of up to
-// kMgRun n-tiles) unit: A's k-slice is staged once, transposed (At[k][j], so a lane's
-// MFMA fragment is one 16-byte read), then the block walks down its n-tiles.  For
-// each tile the next tile's packed dwords and B fragments are loaded into registers
-// while the current tile is computed; every pointer is a per-tile uniform base plus a
-// per-thread 32-bit offset that does not change along the walk.  Units are dealt to
-// the XCDs in contiguous runs (k-tile fastest), so the blocks sharing the lines of a
-// packed row run on one L2.
-constexpr int kMgRun = 16;
-constexpr int kMgAtP = 72;  // u16 pitch of At (16-byte rows)
+// The merge for r <= 64: a unit is one (expert, 256-column k-tile, run of 64-row
+// n-tiles), and each of the block's eight waves walks the run on its own, with no
+// block barrier: LAYOUT 1 [E][K][N] takes 64 n x 32 k per wave and tile, LAYOUT 0
+// [E][N][K] 32 n x 64 k.  The rows of the MFMA's A operand (the adapter's k
+// columns) are permuted so that the 16 accumulators of a lane are 16 consecutive
+// k of one n: its packed codes are one run of 8 bytes, dequantised and summed in
+// registers, and only the bf16 result goes through LDS (wave-private), once, to
+// turn it into 128-byte output runs.  The A fragments stay in registers along the
+// run; the next tile's codes, scales and B fragments are loaded while the current
+// tile is computed.
+// HBM bounds it, and the reads cost more than their share: 32 experts' gate_up at
+// r 16 take 159 us [E][K][N] / 112 us [E][N][K] without the stores, and 251 / 200
+// us with loads that all hit in L2, where the whole takes 358 / 331.  So a unit
+// reads 128 bytes of each packed row (a whole line; 64 bytes per unit: 387 / 343
+// us, codes loaded non-temporally: 517 / 344), and units are dealt to the XCDs
+// in contiguous runs (k-tile fastest), so the blocks that share lines of packed
+// rows and scales run on one L2.  Runs of 8 n-tiles: 16 381 / 341, 4 367 / 321 at
+// r 16 but no better at r 32.  Two to six tiles of loads in flight changed
+// nothing.  Against the form before (64 x 64 tiles by four waves together, the
+// delta as fp32 and the sum as bf16 through LDS, three block barriers per tile):
+// r 16 377 / 368 -> 358 / 331 us, r 32 411 / 404 -> 395 / 358 (1.36 GB, 3.8 / 4.1
+// TB/s).
+constexpr int kMgWaves = 8;     // waves of a block
+constexpr int kMgBK = 32 * kMgWaves;  // k columns of a unit
+constexpr int kMgRun = 8;       // n-tiles of a unit (fewer where the launch has few units)
+constexpr int kMgTP = 72;       // u16 pitch of a wave's result tile (16-byte rows)
+constexpr int kMgUnits = 1024;  // units below which the runs are halved
+typedef af3_u32x4 mg_u32x4_a4 __attribute__((aligned(4)));  // the packed blocks are 4-byte aligned
+typedef __attribute__((ext_vector_type(2))) uint32_t mg_u32x2;
+typedef mg_u32x2 mg_u32x2_a4 __attribute__((aligned(4)));
 
-__global__ __launch_bounds__(256, 4) void lora_merge_kernel(const uint8_t* __restrict__ blocks,
-                                                            const uint8_t* __restrict__ scales,
-                                                            const uint16_t* __restrict__ la,
-                                                            const uint16_t* __restrict__ lb, float s,
-                                                            uint16_t* __restrict__ out, int N, int K, int r,
-                                                            int layout, int n_tiles_n, int n_tiles_k, int n_runs,
-                                                            int n_units, int per_xcd) {
-  __shared__ __attribute__((aligned(16))) uint16_t At[kMgK * kMgAtP];
-  __shared__ __attribute__((aligned(16))) float D[kMgN * kMgDP];
-  __shared__ __attribute__((aligned(16))) uint16_t Mt[kMgN * kMgMP];
+__device__ __forceinline__ void mg_wave_sync() {  // orders a wave's LDS accesses (the LDS keeps their order)
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+// RQ: 16-deep MFMA steps of the rank
+template <int LAYOUT, int RQ>
+__global__ __launch_bounds__(64 * kMgWaves, RQ <= 2 ? 4 : 2) void lora_merge_kernel(
+    const uint8_t* __restrict__ blocks, const uint8_t* __restrict__ scales, const uint16_t* __restrict__ la,
+    const uint16_t* __restrict__ lb, float s, uint16_t* __restrict__ out, int N, int K, int r, int n_tiles_n,
+    int n_tiles_k, int run_tiles, int n_runs, int n_units, int per_xcd) {
+#pragma clang fp contract(off)
+  constexpr int NT = LAYOUT ? 2 : 1, KT = LAYOUT ? 1 : 2;  // 32-wide sub-tiles of a wave along n and k
+  __shared__ __attribute__((aligned(16))) uint16_t lds[kMgWaves][32 * kMgTP];
   const int unit = (int)(blockIdx.x & 7) * per_xcd + (int)(blockIdx.x >> 3);
   if (unit >= n_units || unit >= ((int)(blockIdx.x & 7) + 1) * per_xcd) return;
-  const int kt_i = unit % n_tiles_k;
   const int rest = unit / n_tiles_k;
-  const int run = rest % n_runs;
   const int e = rest / n_runs;
-  const int k0 = kt_i * kMgK;
-  const int t_first = run * kMgRun;
-  const int t_last = min(n_tiles_n, t_first + kMgRun);
+  const int t_first = (rest % n_runs) * run_tiles;
+  const int t_last = min(n_tiles_n, t_first + run_tiles);
   const int G = K >> 5;
-  const int tid = threadIdx.x;
-  const int w = tid >> 6;
-  const int lane = tid & 63;
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c = lane & 31, h = lane >> 5;
+  const int kw = (unit % n_tiles_k) * kMgBK + (LAYOUT ? w * 32 : (w % (kMgWaves / 2)) * 64);  // the wave's first k
+  const int nw = LAYOUT ? 0 : (w / (kMgWaves / 2)) * 32;  // its first n in a tile
+  if (kw >= K) return;
+  uint16_t* const T = lds[w];
 
-  // ---- At[k][j] = A[e][j][k0 + k]
-  {
-    const uint16_t* a_e = la + (int64_t)e * r * K + k0;
-    const int c = tid & 7;
+  // A operand: MFMA row m = 8 j + 4 h + q is k = kw + (LAYOUT 1: 16, else 32) h + 16 t + 4 j + q
+  af3_bf16x8 af[KT][RQ];
 #pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      const int j = h * 32 + (tid >> 3);
-      if (j < r) {
-        af3_u32x4 val = {0u, 0u, 0u, 0u};
-        if (k0 + c * 8 < K) val = *(const af3_u32x4*)(a_e + j * K + c * 8);
+  for (int t = 0; t < KT; ++t) {
+    const int k = kw + ((c >> 2) & 1) * (LAYOUT ? 16 : 32) + t * 16 + 4 * (c >> 3) + (c & 3);
+    const uint16_t* a_k = la + (int64_t)e * r * K + min(k, K - 1);  // columns past K are not stored
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          At[(c * 8 + 2 * i) * kMgAtP + j] = (uint16_t)(val[i] & 0xFFFFu);
-          At[(c * 8 + 2 * i + 1) * kMgAtP + j] = (uint16_t)(val[i] >> 16);
-        }
-      }
+    for (int q = 0; q < RQ; ++q) {
+      const int j = q * 16 + h * 8;  // 8 reduction indices (r % 8 == 0)
+      uint32_t v[4] = {0u, 0u, 0u, 0u};
+      if (j < r)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+          v[i] = (uint32_t)a_k[(int64_t)(j + 2 * i) * K] | ((uint32_t)a_k[(int64_t)(j + 2 * i + 1) * K] << 16);
+      af[t][q] = __builtin_bit_cast(af3_bf16x8, (af3_u32x4){v[0], v[1], v[2], v[3]});
     }
   }
 
-  // per-thread offsets, fixed along the walk
-  const int kl = (tid & 7) * 8;            // 8 consecutive k of rows p*32 + tid/8
-  const bool k_live = k0 + kl < K;
-  const int kcl = (w & 1) * 32 + (lane & 31);
-  const int nsub = (w >> 1) * 32 + (lane & 31);
-  const int jh = (lane >> 5) * 8;
-  uint32_t off_b[2], off_s[2];
+  // a lane's codes: LAYOUT 1 half a block (16 k) of rows c and 32 + c, else the block (32 k) of row c
+  const int kb = min((kw >> 5) + (LAYOUT ? 0 : h), G - 1);
+  struct Tile {
+    uint32_t v[4], sc[NT];
+    af3_u32x4 b[NT][RQ];
+  };
+  auto fetch = [&](int ti, Tile& d) {
 #pragma unroll
-  for (int p = 0; p < 2; ++p) {
-    const int nl = p * 32 + (tid >> 3);
-    off_b[p] = (uint32_t)(nl * G * 16 + (kl >> 1));
-    off_s[p] = (uint32_t)(nl * G + (kl >> 5));
-  }
-  const uint32_t off_lb = (uint32_t)(nsub * r + jh);
-
-  uint32_t v[2], sc[2];
-  af3_u32x4 bv[4];
-  auto fetch = [&](int ti, uint32_t v_[2], uint32_t sc_[2], af3_u32x4 bv_[4]) {
-    const int n0 = ti * kMgN;
-    const int64_t row0 = (int64_t)e * N + n0;
-    const uint8_t* bt = blocks + (row0 * G + (k0 >> 5)) * 16;
-    const uint8_t* st = scales + row0 * G + (k0 >> 5);
+    for (int t = 0; t < NT; ++t) {
+      const int64_t row = (int64_t)e * N + min(ti * kMgN + nw + t * 32 + c, N - 1);  // rows past N are not stored
+      const int64_t grp = row * G + kb;
+      if constexpr (LAYOUT) {
+        const mg_u32x2 x = *(const mg_u32x2_a4*)(blocks + grp * 16 + h * 8);
+        d.v[2 * t] = x[0];
+        d.v[2 * t + 1] = x[1];
+      } else {
+        const af3_u32x4 x = *(const mg_u32x4_a4*)(blocks + grp * 16);
 #pragma unroll
-    for (int p = 0; p < 2; ++p) {
-      v_[p] = 0u;
-      sc_[p] = 0u;
-      if (n0 + p * 32 + (tid >> 3) < N && k_live) {
-        v_[p] = __builtin_nontemporal_load((const uint32_t*)(bt + off_b[p]));
-        sc_[p] = st[off_s[p]];
+        for (int i = 0; i < 4; ++i) d.v[i] = x[i];
       }
-    }
-    const uint16_t* lt = lb + row0 * r;
-    const bool n_ok = n0 + nsub < N;
+      d.sc[t] = scales[grp];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      bv_[q] = (af3_u32x4){0u, 0u, 0u, 0u};
-      if (q * 16 + jh < r && n_ok) bv_[q] = *(const af3_u32x4*)(lt + off_lb + q * 16);
+      for (int q = 0; q < RQ; ++q)  // no branch: lanes past the rank load its last indices and zero them before use
+        d.b[t][q] = *(const af3_u32x4*)(lb + row * r + min(q * 16 + h * 8, r - 8));
     }
   };
-  fetch(t_first, v, sc, bv);
-
-  for (int ti = t_first; ti < t_last; ++ti) {
+  const bool tail_rank = r < RQ * 16;
+  // one tile from `cur`, the next one's operands into `nxt`. WHOLE: every store
+  // unconditional, so that the compiler's wait for `nxt` counts them and leaves
+  // them in flight
+  auto step = [&](auto whole_c, int ti, Tile& cur, Tile& nxt) {
+    constexpr bool WHOLE = decltype(whole_c)::value;
     const int n0 = ti * kMgN;
-    // consume the registers the previous fetch filled before the next fetch is issued,
-    // so that no wait for the new loads is needed before the end of this tile
-    uint32_t qd[2][4];
+    fetch(min(ti + 1, t_last - 1), nxt);
+    if (tail_rank) {
 #pragma unroll
-    for (int p = 0; p < 2; ++p) af3_dequant_u32(v[p], sc[p], qd[p]);
+      for (int q = 0; q < RQ; ++q)
 #pragma unroll
-    for (int q = 0; q < 4; ++q) asm volatile("" : "+v"(bv[q]));
-    uint32_t vn[2] = {0u, 0u}, scn[2] = {0u, 0u};
-    af3_u32x4 bvn[4] = {};
-    if (ti + 1 < t_last) fetch(ti + 1, vn, scn, bvn);
-    __syncthreads();  // At staged (first tile); the previous tile's reads of D and Mt are done
-
-    af3_f32x16 acc;
+        for (int t = 0; t < NT; ++t)
 #pragma unroll
-    for (int i = 0; i < 16; ++i) acc[i] = 0.f;
-#pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      if (q * 16 >= r) break;
-      af3_u32x4 bw = {0u, 0u, 0u, 0u};
-      if (q * 16 + jh < r) bw = *(const af3_u32x4*)(At + kcl * kMgAtP + q * 16 + jh);
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(af3_bf16x8, bv[q]),
-                                                    __builtin_bit_cast(af3_bf16x8, bw), acc, 0, 0, 0);
+          for (int i = 0; i < 4; ++i) cur.b[t][q][i] = q * 16 + h * 8 < r ? cur.b[t][q][i] : 0u;
     }
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-      const int row = (w >> 1) * 32 + (i >> 2) * 8 + (lane >> 5) * 4 + (i & 3);
-      D[row * kMgDP + kcl] = acc[i] * s;
-    }
-    __syncthreads();
-
+    for (int u = 0; u < 2; ++u) {  // the two 32 x 32 sub-tiles
+      af3_f32x16 acc;
 #pragma unroll
-    for (int p = 0; p < 2; ++p) {
-      const int nl = p * 32 + (tid >> 3);
-      const bool live = n0 + nl < N && k_live;
-      uint32_t m[4] = {0u, 0u, 0u, 0u};
-      if (live) {
-        const float4* d4 = (const float4*)(D + nl * kMgDP + kl);
+      for (int i = 0; i < 16; ++i) acc[i] = 0.f;
 #pragma unroll
-        for (int c = 0; c < 2; ++c) {
-          const float4 d = d4[c];
-          const uint32_t lo = qd[p][2 * c], hi = qd[p][2 * c + 1];
-          m[2 * c] = af3_pack_bf16x2(af3_bf16_to_f32(lo & 0xFFFFu) + d.x, af3_bf16_to_f32(lo >> 16) + d.y);
-          m[2 * c + 1] = af3_pack_bf16x2(af3_bf16_to_f32(hi & 0xFFFFu) + d.z, af3_bf16_to_f32(hi >> 16) + d.w);
-        }
-      }
-      if (layout == 0) {
-        if (live)
-          __builtin_nontemporal_store((af3_u32x4){m[0], m[1], m[2], m[3]},
-                                      (af3_u32x4*)(out + ((int64_t)e * N + n0) * K + k0 + (uint32_t)(nl * K + kl)));
-      } else {
-        uint32_t* mrow = (uint32_t*)(Mt + nl * kMgMP + kl);
-#pragma unroll
-        for (int c = 0; c < 4; ++c) mrow[c] = m[c];
-      }
-    }
-    if (layout != 0) {
-      __syncthreads();
-      const int nt = (tid & 7) * 8;
-      uint16_t* ot = out + ((int64_t)e * K + k0) * N + n0;
+      for (int q = 0; q < RQ; ++q)
+        acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[LAYOUT ? 0 : u][q],
+                                                      __builtin_bit_cast(af3_bf16x8, cur.b[LAYOUT ? u : 0][q]), acc, 0,
+                                                      0, 0);
+      uint32_t m[8];
 #pragma unroll
       for (int p = 0; p < 2; ++p) {
-        const int kt = p * 32 + (tid >> 3);
-        if (k0 + kt >= K) break;
-        uint32_t t4[4];
+        uint32_t d[4];
+        af3_dequant_u32(cur.v[2 * u + p], cur.sc[LAYOUT ? u : 0], d);
 #pragma unroll
-        for (int c = 0; c < 4; ++c)
-          t4[c] = (uint32_t)Mt[(nt + 2 * c) * kMgMP + kt] | ((uint32_t)Mt[(nt + 2 * c + 1) * kMgMP + kt] << 16);
-        uint16_t* o = ot + (uint32_t)(kt * N + nt);
-        if ((N & 7) == 0 && n0 + nt + 8 <= N) {
-          __builtin_nontemporal_store((af3_u32x4){t4[0], t4[1], t4[2], t4[3]}, (af3_u32x4*)o);
-        } else {
-          for (int c = 0; c < 8 && n0 + nt + c < N; ++c) o[c] = (uint16_t)(t4[c >> 1] >> (16 * (c & 1)));
+        for (int i = 0; i < 4; ++i) {
+          const float lo = acc[8 * p + 2 * i] * s, hi = acc[8 * p + 2 * i + 1] * s;
+          m[4 * p + i] = af3_pack_bf16x2(af3_bf16_to_f32(d[i] & 0xFFFFu) + lo, af3_bf16_to_f32(d[i] >> 16) + hi);
         }
       }
-    }
+      if constexpr (LAYOUT) {  // T[k][n]
+        uint16_t* const col = T + h * 16 * kMgTP + u * 32 + c;
 #pragma unroll
-    for (int p = 0; p < 2; ++p) {
-      v[p] = vn[p];
-      sc[p] = scn[p];
+        for (int i = 0; i < 8; ++i) {
+          col[2 * i * kMgTP] = (uint16_t)m[i];
+          col[(2 * i + 1) * kMgTP] = (uint16_t)(m[i] >> 16);
+        }
+      } else {  // T[n][k]
+        af3_u32x4* const row = (af3_u32x4*)(T + c * kMgTP + h * 32 + u * 16);
+        row[0] = (af3_u32x4){m[0], m[1], m[2], m[3]};
+        row[1] = (af3_u32x4){m[4], m[5], m[6], m[7]};
+      }
     }
+    mg_wave_sync();
+    const int tr = lane >> 3, tc = (lane & 7) * 8;
 #pragma unroll
-    for (int q = 0; q < 4; ++q) bv[q] = bvn[q];
-  }
+    for (int i = 0; i < 4; ++i) {
+      const int rr = i * 8 + tr;
+      const af3_u32x4 v = *(const af3_u32x4*)(T + rr * kMgTP + tc);
+      if constexpr (LAYOUT) {
+        uint16_t* const o = out + ((int64_t)e * K + kw + rr) * N + n0 + tc;
+        if (WHOLE || (N & 7) == 0) {
+          if (WHOLE || n0 + tc < N) __builtin_nontemporal_store(v, (af3_u32x4*)o);
+        } else {
+          for (int x = 0; x < 8; ++x)
+            if (n0 + tc + x < N) o[x] = (uint16_t)(v[x >> 1] >> (16 * (x & 1)));
+        }
+      } else {
+        const int n = n0 + nw + rr;
+        if (WHOLE || (n < N && kw + tc < K))
+          __builtin_nontemporal_store(v, (af3_u32x4*)(out + ((int64_t)e * N + n) * K + kw + tc));
+      }
+    }
+    mg_wave_sync();
+  };
+  auto walk = [&](auto whole_c) {
+    Tile a, b;
+    fetch(t_first, a);
+    for (int ti = t_first;;) {
+      step(whole_c, ti, a, b);
+      if (++ti >= t_last) break;
+      step(whole_c, ti, b, a);
+      if (++ti >= t_last) break;
+    }
+  };
+  if (t_last * kMgN <= N && (LAYOUT ? (N & 7) == 0 : kw + 64 <= K))
+    walk(std::true_type{});
+  else
+    walk(std::false_type{});
 }
 
 }  // namespace
@@ -398,13 +411,27 @@ extern "C" int af3_mxfp4_lora_merge(const uint8_t* blocks, const uint8_t* scales
   const int64_t per_xcd = af3_cdiv(tiles, 8);
   // resident blocks per XCD: 32 CUs x 6 blocks of 26 KB LDS
   if (r <= 64) {
-    const int runs = (int)af3_cdiv(ntn, kMgRun);
-    const int64_t units = (int64_t)E * runs * ntk;
+    const int nk = (int)af3_cdiv(K, kMgBK);
+    int run = kMgRun;  // shorter runs while the launch would leave CUs idle
+    while (run > 2 && (int64_t)E * af3_cdiv(ntn, run) * nk < kMgUnits) run /= 2;
+    const int runs = (int)af3_cdiv(ntn, run);
+    const int64_t units = (int64_t)E * runs * nk;
     AF3_REQUIRE(units <= 0x7ffffff0LL && (int64_t)kMgN * N <= 0x7fffffffLL && (int64_t)kMgK * N <= 0x7fffffffLL,
                 "mxfp4_lora_merge: tensor too large");
     const int upx = (int)af3_cdiv(units, 8);
-    hipLaunchKernelGGL(lora_merge_kernel, dim3((unsigned)(8 * upx)), dim3(256), 0, stream, blocks, scales, lora_a,
-                       lora_b, scaling, out, N, K, r, layout, ntn, ntk, runs, (int)units, upx);
+#define AF3_MG(lay, rq)                                                                                        \
+  hipLaunchKernelGGL((lora_merge_kernel<lay, rq>), dim3((unsigned)(8 * upx)), dim3(64 * kMgWaves), 0, stream,  \
+                     blocks, scales, lora_a, lora_b, scaling, out, N, K, r, ntn, nk, run, runs, (int)units, upx)
+#define AF3_MGR(lay)              \
+  do {                            \
+    if (r <= 16) AF3_MG(lay, 1);  \
+    else if (r <= 32) AF3_MG(lay, 2); \
+    else AF3_MG(lay, 4);          \
+  } while (0)
+    if (layout) AF3_MGR(1);
+    else AF3_MGR(0);
+#undef AF3_MGR
+#undef AF3_MG
   } else {
     const int bpx = (int)(per_xcd < kMgBlocksPerXcd ? per_xcd : kMgBlocksPerXcd);
     hipLaunchKernelGGL(lora_merge_generic_kernel, dim3((unsigned)(8 * bpx)), dim3(256), 0, stream, blocks, scales,

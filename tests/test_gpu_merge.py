@@ -71,6 +71,22 @@ def test_merge_within_one_step(dev, E, N, G, r, layout):
     _check_close(got, blocks, scales, A, B, s, layout, 2e-3)
 
 
+# edges of the 64 x 256 tiles: one row, one block, a row past a tile, K = 32 to 224 mod 256, ragged N (no 16-byte
+# stores in "hf"), every rank step, runs of several tiles; off = blocks at a 4-byte aligned address only
+@pytest.mark.parametrize("E,N,G,r,off", [(1, 1, 1, 8, 0), (2, 65, 4, 16, 4), (1, 200, 7, 24, 0), (1, 129, 9, 32, 8),
+                                         (1, 1100, 3, 48, 12), (2, 64, 6, 56, 0), (3, 72, 13, 64, 4)])
+@pytest.mark.parametrize("layout", ["rows", "hf"])
+def test_merge_tile_edges(dev, E, N, G, r, off, layout):
+    blocks, scales, A, B = _inputs(E, N, G, r, seed=E * 100 + N + r)
+    print(f"merge edges E,N,G,r,off={(E, N, G, r, off)} layout={layout}", flush=True)
+    store = torch.zeros(blocks.numel() + 16, dtype=torch.uint8, device=dev)
+    b = store[off:off + blocks.numel()].view(blocks.shape)
+    b.copy_(blocks)
+    got = kernels.mxfp4_lora_merge(b, scales.to(dev), A.to(dev), B.to(dev), 32.0 / r, layout)
+    torch.cuda.synchronize()
+    _check_close(got, blocks, scales, A, B, 32.0 / r, layout, 2e-3 + 2.0 / got.numel())
+
+
 @pytest.mark.parametrize("layout", ["rows", "hf"])
 def test_merge_exact_sums_every_scale_byte(dev, layout):
     # adapters on a 2^-4 / 2^-3 grid: the r-term sum is exact in fp32 in any order,
