@@ -151,5 +151,7 @@ def ptr(t) -> int | None:
 
 def stream_of(device: torch.device) -> int:
     """The device's current stream as a hipStream_t, without a Stream object around it."""
+    if device.type != "cuda":  # a host pointer would follow
+        raise ValueError(f"Expected a cuda device, but got: {device}")
     index = device.index
     return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if index is None else index)

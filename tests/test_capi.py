@@ -61,3 +61,13 @@ def test_product_path_has_no_oracle_dependency():
     pkg = ROOT / "agent-factory-3_amd" / "agent_factory_3_amd"
     for f in pkg.glob("*.py"):
         assert "oracle" not in re.findall(r"^\s*(?:from|import)\s+(\w+)", f.read_text(), re.M), f.name
+
+
+def test_stream_of_refuses_a_host_device():
+    # the stream lookup is what stops host tensors from reaching a kernel as pointers
+    import pytest
+    import torch
+
+    from agent_factory_3_amd import _capi
+    with pytest.raises(ValueError, match="cuda device"):
+        _capi.stream_of(torch.device("cpu"))
