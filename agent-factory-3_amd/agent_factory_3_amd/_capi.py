@@ -30,6 +30,7 @@ _SIGNATURES = {
     "af3_swiglu_bwd": (_i32, [_p, _i64, _p, _p, _i64, _p, _i64, _i64, _i64, _f32, _f32, _p]),
     "af3_swiglu_bwd_raw": (_i32, [_p, _i64, _p, _i64, _p, _i64, _i64, _i64, _f32, _f32, _p]),
     "af3_routing_workspace_bytes": (_sz, [_i64, _i32, _i32]),
+    "af3_routing_count_rows": (_sz, [_i64, _i32, _i32]),
     "af3_routing_replay": (_i32, [_p, _i64, _p, _i64, _i32, _i32, _p, _p, _p, _p, _p, _p, _sz, _p]),
     "af3_routing_topk": (_i32, [_p, _i64, _i64, _i32, _i32, _p, _p, _p, _p, _p, _p, _sz, _p]),
     "af3_routing_scratch_bytes": (_sz, []),

@@ -243,7 +243,7 @@ constexpr int kPlanMaxTopkE = 256;    // experts of the 16-lane top-k (16 logits
 constexpr int kPlanSmallR = 4096;     // entries of the one-block plan
 constexpr int kPlanSmallTopkT = 256;  // tokens whose top-k the one-block plan takes along (64 per pass)
 constexpr int kPlanSmallCnt = 16384;  // (64-entry group, expert) counters of the one-block plan (64 KB)
-constexpr int kPlanTokens = 64;       // tokens per chunk of the three-launch plan (one pass of 16-lane groups)
+constexpr int kPlanTokens = 64;       // tokens of one pass of 16-lane groups (three-launch plan)
 constexpr int kPlanMaxBm = 8;
 
 // tile maps and work orders to make (n_bm = 0: none); orders for the first n_order sizes
@@ -550,23 +550,23 @@ __global__ __launch_bounds__(1024) void plan_small_kernel(const uint16_t* __rest
   plan_maps(m, E, counts);
 }
 
-// ids and weights (MODE as above) and the expert counts of each chunk of kPlanTokens tokens: counts[chunk][E]
+// ids and weights (MODE as above) and the expert counts of each chunk of `chunk` tokens: counts[chunk][E]
 template <int MODE>
 __global__ __launch_bounds__(1024) void token_hist_kernel(const uint16_t* __restrict__ logits, int64_t ld,
                                                           const int32_t* __restrict__ idx, int64_t T, int E, int K,
-                                                          int32_t* __restrict__ ids, uint16_t* __restrict__ scal,
-                                                          int32_t* __restrict__ counts) {
+                                                          int chunk, int32_t* __restrict__ ids,
+                                                          uint16_t* __restrict__ scal, int32_t* __restrict__ counts) {
   __shared__ int32_t sh[kPlanMaxE];
   const int t = threadIdx.x;
   for (int e = t; e < E; e += 1024) sh[e] = 0;
   __syncthreads();
-  const int64_t t0 = (int64_t)blockIdx.x * kPlanTokens;
+  const int64_t t0 = (int64_t)blockIdx.x * chunk;
   if constexpr (MODE == 2) {
-    const int64_t hi = min((t0 + kPlanTokens) * K, T * K);
+    const int64_t hi = min((t0 + chunk) * K, T * K);
     for (int64_t i = t0 * K + t; i < hi; i += 1024)
       if (ids[i] >= 0) atomicAdd(&sh[ids[i]], 1);
   } else {
-    for (int q = 0; q < kPlanTokens; q += 64) {
+    for (int q = 0; q < chunk; q += kPlanTokens) {
       const int64_t tok = t0 + q + (t >> 4);
       int32_t e;
       uint16_t w;
@@ -632,8 +632,9 @@ __global__ __launch_bounds__(1024) void plan_scan_kernel(int32_t* __restrict__ c
 
 // stable scatter of chunk blockIdx.x into expert-sorted order, and the slots past the valid entries
 __global__ __launch_bounds__(256) void plan_scatter_kernel(const int32_t* __restrict__ ids,
-                                                            const uint16_t* __restrict__ scal, int64_t R, int E, int K,
-                                                            int ebits, const int32_t* __restrict__ offs,
+                                                            const uint16_t* __restrict__ scal, int64_t R, int E,
+                                                            int chunk_entries, int ebits,
+                                                            const int32_t* __restrict__ offs,
                                                             const int32_t* __restrict__ counts,
                                                             int32_t* __restrict__ topk_indx,
                                                             int32_t* __restrict__ gate_indx,
@@ -643,8 +644,8 @@ __global__ __launch_bounds__(256) void plan_scatter_kernel(const int32_t* __rest
   const int t = threadIdx.x, wave = t >> 6;
   for (int e = t; e < E; e += 256) base[e] = offs[e] + counts[(int64_t)blockIdx.x * E + e];
   const int64_t valid = offs[E];
-  const int64_t lo = (int64_t)blockIdx.x * kPlanTokens * K;
-  const int64_t hi = min(lo + (int64_t)kPlanTokens * K, R);
+  const int64_t lo = (int64_t)blockIdx.x * chunk_entries;
+  const int64_t hi = min(lo + chunk_entries, R);
   for (int64_t i0 = lo; i0 < hi; i0 += 256) {
     const int64_t i = i0 + t;
     const int e = i < hi ? ids[i] : -1;
@@ -813,16 +814,34 @@ __global__ __launch_bounds__(1024) void tile_order_kernel(const int32_t* __restr
 
 }  // namespace
 
+// What a batch keeps in the workspace: ids [R] at 0, weights [R], then one row
+// of E counts per chunk.  The size queries and the launches both take it from
+// here.  A chunk of the plan holds at least as many entries as the older
+// chain's kChunk (64 tokens of 4 entries or more, 128 of 2 or 3, 256 of one), so
+// the plan never needs more than the older chain did.
+struct RoutingLayout {
+  int chunk_tokens;  // tokens per chunk (plan)
+  int64_t rows;      // chunks
+  size_t scal, counts, bytes;
+};
+static RoutingLayout routing_layout(int64_t T, int E, int K) {
+  const int64_t R = T * K;
+  const auto up = [](size_t b) { return (b + 255) & ~(size_t)255; };
+  RoutingLayout l;
+  l.chunk_tokens = kPlanTokens * (K >= 4 ? 1 : K >= 2 ? 2 : 4);
+  l.rows = E <= kPlanMaxE ? af3_cdiv(T, l.chunk_tokens) : af3_cdiv(R, kChunk);
+  l.scal = up((size_t)R * 4);
+  l.counts = up(l.scal + (size_t)R * 2);
+  l.bytes = l.counts + (size_t)l.rows * E * 4 + 256;
+  return l;
+}
+
 extern "C" size_t af3_routing_workspace_bytes(int64_t n_tokens, int n_expts_tot, int n_expts_act) {
-  int64_t R = n_tokens * n_expts_act;
-  int64_t n_chunks = af3_cdiv(R, kChunk);
-  size_t b = 0;
-  b += (size_t)R * 4;                       // ids
-  b = (b + 255) & ~(size_t)255;
-  b += (size_t)R * 2;                       // scal
-  b = (b + 255) & ~(size_t)255;
-  b += (size_t)n_chunks * n_expts_tot * 4;  // counts
-  return b + 256;
+  return routing_layout(n_tokens, n_expts_tot, n_expts_act).bytes;
+}
+
+extern "C" size_t af3_routing_count_rows(int64_t n_tokens, int n_expts_tot, int n_expts_act) {
+  return (size_t)routing_layout(n_tokens, n_expts_tot, n_expts_act).rows;
 }
 
 extern "C" size_t af3_routing_plan_workspace_bytes(int64_t n_tokens, int n_expts_tot, int n_expts_act, int topk);
@@ -838,8 +857,8 @@ static bool plan_one_block(bool topk, int64_t T, int E, int K) {
 // E <= 1024: the merged chain, with the tile maps of `m` where it asks for any
 static int routing_plan(bool topk, const uint16_t* logits, int64_t ld, const int32_t* expt_indx, int64_t T, int E, int K,
                         uint16_t* gate_scal, int32_t* hist, int32_t* topk_indx, int32_t* gate_indx,
-                        int32_t* token_offs_raw, int32_t* ids, uint16_t* scal, int32_t* counts, const PlanMaps& m,
-                        hipStream_t stream) {
+                        int32_t* token_offs_raw, int32_t* ids, uint16_t* scal, int32_t* counts,
+                        const RoutingLayout& lay, const PlanMaps& m, hipStream_t stream) {
   const int64_t R = T * K;
   const int ebits = E > 1 ? 32 - __builtin_clz((unsigned)(E - 1)) : 1;
   const bool lane_topk = topk && E <= kPlanMaxTopkE;
@@ -861,10 +880,10 @@ static int routing_plan(bool topk, const uint16_t* logits, int64_t ld, const int
 #undef AF3_PLAN
     return af3::check_launch("routing/plan");
   }
-  const int n_chunks = (int)af3_cdiv(T, kPlanTokens);
+  const int n_chunks = (int)lay.rows;
 #define AF3_TOK(md)                                                                                          \
   hipLaunchKernelGGL(token_hist_kernel<md>, dim3(n_chunks), dim3(1024), 0, stream, logits, ld, expt_indx, T, E, K, \
-                     ids, scal, counts)
+                     lay.chunk_tokens, ids, scal, counts)
   if (mode == 0) AF3_TOK(0);
   else if (mode == 1) AF3_TOK(1);
   else AF3_TOK(2);
@@ -876,8 +895,8 @@ static int routing_plan(bool topk, const uint16_t* logits, int64_t ld, const int
                      m);
   rc = af3::check_launch("routing/scan");
   if (rc) return rc;
-  hipLaunchKernelGGL(plan_scatter_kernel, dim3(n_chunks), dim3(256), 0, stream, ids, scal, R, E, K, ebits,
-                     token_offs_raw, counts, topk_indx, gate_indx, gate_scal);
+  hipLaunchKernelGGL(plan_scatter_kernel, dim3(n_chunks), dim3(256), 0, stream, ids, scal, R, E,
+                     lay.chunk_tokens * K, ebits, token_offs_raw, counts, topk_indx, gate_indx, gate_scal);
   return af3::check_launch("routing/scatter");
 }
 
@@ -898,20 +917,16 @@ static int routing_common(bool topk, const uint16_t* logits, int64_t ld, const i
   const int64_t R = T * K;
   AF3_REQUIRE(R < 0x7fffffffLL, "routing: T*K too large");
   char* ws = (char*)workspace;
-  size_t o = 0;
-  int32_t* ids = (int32_t*)(ws + o);
-  o += (size_t)R * 4;
-  o = (o + 255) & ~(size_t)255;
-  uint16_t* scal = (uint16_t*)(ws + o);
-  o += (size_t)R * 2;
-  o = (o + 255) & ~(size_t)255;
-  int32_t* counts = (int32_t*)(ws + o);
+  const RoutingLayout lay = routing_layout(T, E, K);
+  int32_t* ids = (int32_t*)ws;
+  uint16_t* scal = (uint16_t*)(ws + lay.scal);
+  int32_t* counts = (int32_t*)(ws + lay.counts);
   if (E <= kPlanMaxE) {
     const PlanMaps none{};
     return routing_plan(topk, logits, ld, expt_indx, T, E, K, gate_scal, hist, topk_indx, gate_indx, token_offs_raw,
-                        ids, scal, counts, maps ? *maps : none, stream);
+                        ids, scal, counts, lay, maps ? *maps : none, stream);
   }
-  const int n_chunks = (int)af3_cdiv(R, kChunk);
+  const int n_chunks = (int)lay.rows;
 
   if (T > 0) {
     dim3 g((unsigned)af3_cdiv(T, 128));

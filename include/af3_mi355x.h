@@ -58,8 +58,11 @@ int af3_swiglu_bwd_raw(const uint16_t* grad_out, int64_t ld_grad, const uint16_t
                        uint16_t* grad_gu, int64_t ld_gu, int64_t M, int64_t N, float alpha, float limit,
                        void* stream);
 
-/* Workspace bytes needed by af3_routing_replay / af3_routing_topk. */
+/* Workspace bytes needed by af3_routing_replay / af3_routing_topk: int32 ids and
+ * bf16 weights of the T*K entries, then af3_routing_count_rows rows of n_expts_tot
+ * int32 counts (one row per chunk of tokens), each part 256-byte aligned. */
 size_t af3_routing_workspace_bytes(int64_t n_tokens, int n_expts_tot, int n_expts_act);
+size_t af3_routing_count_rows(int64_t n_tokens, int n_expts_tot, int n_expts_act);
 
 /* Routing from given expert ids.  Replaces quantization.py:593-636
  * (routing_replay).  logits [T][ld] bf16, expt_indx [T][K] int32 ->

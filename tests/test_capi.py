@@ -57,6 +57,29 @@ def test_noalloc_routing_rejects_shapes_beyond_its_scratch():
         _capi.call("af3_routing_replay_noalloc", 1, E, 1, T, E, K, 1, 1, 1, 1, 1, None)
 
 
+@pytest.mark.parametrize("E", [1, 3, 32, 64, 128, 1024, 1025])
+def test_routing_workspace_covers_its_count_rows(E):
+    """The reported workspace holds the ids, the weights and every count row the
+    launches write, for any number of experts per token, and is never more than
+    one row per 256 entries asks for (sizes a caller kept, the built-in array)."""
+    from agent_factory_3_amd import _capi
+    if not _capi.lib_path().exists():
+        pytest.skip("library not built")
+    lib = _capi.load()
+    up = lambda n: (n + 255) // 256 * 256  # noqa: E731
+    for K in range(1, min(E, 16) + 1):
+        for T in (0, 1, 63, 64, 65, 255, 257, 300, 512, 4096, 4097, 8191, 65537, 500000):
+            rows = int(lib.af3_routing_count_rows(T, E, K))
+            head = up(up(4 * T * K) + 2 * T * K)
+            assert (T + 255) // 256 <= rows <= (T * K + 255) // 256
+            assert _capi.workspace_bytes(T, E, K) >= head + 4 * rows * E
+            assert _capi.workspace_bytes(T, E, K) <= head + (T * K + 255) // 256 * E * 4 + 256
+            for topk in (0, 1):
+                n = int(lib.af3_routing_plan_workspace_bytes(T, E, K, topk))
+                one_block = T * K <= 4096 and (not topk or E > 256 or T <= 256)
+                assert n == _capi.workspace_bytes(T, E, K) or (n == 0 and one_block)
+
+
 def test_product_path_has_no_oracle_dependency():
     pkg = ROOT / "agent-factory-3_amd" / "agent_factory_3_amd"
     for f in pkg.glob("*.py"):

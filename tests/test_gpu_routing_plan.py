@@ -3,6 +3,8 @@
 one-block limit, chunk edges of the three-launch form, the smallest and largest
 expert and slot counts, dropped ids, and logits with equal, -0, infinite and NaN
 entries; every index, tile map and work order bit-exact."""
+import ctypes
+
 import pytest
 import torch
 
@@ -100,6 +102,41 @@ def test_entry_points_agree(dev):
                        _capi.stream_of(torch.device(dev)))
             assert torch.equal(o[0], rd.expt_hist) and torch.equal(o[1], gi.src_indx)
             assert torch.equal(o[2], gi.dst_indx) and torch.equal(o[3], rd.expt_data.token_offs_raw)
+
+
+@pytest.mark.parametrize("T,E,K", [(8191, 64, 1), (300, 32, 1), (4096, 32, 2), (512, 1024, 3), (1403, 257, 3),
+                                   (1100, 128, 4), (700, 256, 16)])
+def test_workspace_is_not_exceeded(dev, T, E, K):
+    """Every entry point stays within a workspace of exactly the queried size (bytes behind it unchanged)."""
+    g = torch.Generator().manual_seed(T + E + K)
+    logits = torch.randn(T, E, generator=g).to(torch.bfloat16)
+    ids = torch.rand(T, E, generator=g).topk(K, dim=1).indices.to(torch.int32)
+    lib = _capi.load()
+    ld, idd = logits.to(dev), ids.to(dev)
+    for name in ("af3_routing_topk", "af3_routing_replay", "af3_routing_plan"):
+        for topk in (0, 1):
+            if (name.endswith("topk") and not topk) or (name.endswith("replay") and topk):
+                continue
+            ref = O.routing_topk(logits, K) if topk else O.routing_replay(logits, ids, K)
+            plan = name.endswith("plan")
+            n = int(lib.af3_routing_plan_workspace_bytes(T, E, K, topk)) if plan else _capi.workspace_bytes(T, E, K)
+            ws = torch.full((2 * n + (1 << 20),), 0xA5, dtype=torch.uint8, device=dev)   # room behind the workspace
+            o = [torch.empty(m, dtype=torch.int32, device=dev) for m in (E, T * K, T * K, E + 1)]
+            gs = torch.empty(T * K, dtype=torch.bfloat16, device=dev)
+            outs = (gs.data_ptr(), *[t.data_ptr() for t in o])
+            tail = (ws.data_ptr(), n, _capi.stream_of(torch.device(dev)))
+            if plan:
+                mt = R.max_tiles(T * K, E, 128)
+                pad = torch.empty(E + 1, dtype=torch.int32, device=dev)
+                maps = torch.empty(2, mt, dtype=torch.int32, device=dev)
+                _capi.call(name, ld.data_ptr(), E, idd.data_ptr(), topk, T, E, K, *outs, (ctypes.c_int32 * 1)(128), 1,
+                           1, mt, pad.data_ptr(), maps[0].data_ptr(), maps[1].data_ptr(), *tail)
+            else:
+                _capi.call(name, ld.data_ptr(), E, *(() if topk else (idd.data_ptr(),)), T, E, K, *outs, *tail)
+            torch.cuda.synchronize()
+            assert (ws[n:] == 0xA5).all(), name
+            assert torch.equal(o[1].cpu(), ref["topk_indx"]) and torch.equal(o[0].cpu(), ref["hist"].to(torch.int32))
+            assert torch.equal(o[2].cpu(), ref["gate_indx"])
 
 
 @pytest.mark.parametrize("T,H,E", [(1, 64, 1), (63, 128, 33), (64, 320, 64), (65, 384, 65), (129, 2880, 129),
