@@ -268,12 +268,13 @@ def mxfp4_tile_dx_scales(scales):
     return out
 
 
-def _short_block_m(ed, rows, E, N, K, trans_w, off32):
+def _short_block_m(ed, rows, E, N, K, trans_w, off32, scales_al16=True):
     """The short-tile kernels' map (32 or 64 rows) for a launch of ``rows`` rows
     over E experts, or 0: they need few rows per expert, the map (made with the
-    routing), 32-bit offsets, and whole 320-deep (forward) k-groups."""
+    routing), 32-bit offsets, and (forward) whole 320-deep k-groups and scales at
+    a 16-byte aligned address."""
     if not GEMM_TILE.get("short", True) or not off32 or N % 64 or N * K // 2 >= 1 << 32 \
-            or (not trans_w and (K % 320 or K > 3072)):
+            or (not trans_w and (K % 320 or K > 3072 or not scales_al16)):
         return 0
     for lim, bm in DX_SHORT_ROWS if trans_w else FWD_SHORT_ROWS:
         if rows <= lim * E and bm in ed.block_pid_map and bm in ed.gemm_order:
@@ -326,7 +327,7 @@ def moe_rows(x, blocks, scales, bias, routing_data, gather_indx=None, gammas=Non
         elif trans_w and GEMM_TILE["tile_cfg"] % 100 in (0, 28):
             bm = GEMM_TILE.get("dx_block_m", 128)
         if GEMM_TILE["tile_cfg"] == 0 and bm == 128:
-            bm = _short_block_m(ed, R, E, N, K, trans_w, off32) or bm
+            bm = _short_block_m(ed, R, E, N, K, trans_w, off32, scales.data_ptr() % 16 == 0) or bm
     pid_map = gemm_order_for(ed, bm) if GEMM_TILE.get("order", True) else None
     if pid_map is None:
         pid_map = ed.block_pid_map[bm]

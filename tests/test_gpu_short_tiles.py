@@ -124,6 +124,33 @@ def test_map_choice(dev):
     assert 32 not in big.block_pid_map and Q._short_block_m(big, 100, 16, 5760, 2880, False, True) == 0
 
 
+@pytest.mark.parametrize("off", [1, 8])
+def test_scales_at_an_unaligned_address(dev, monkeypatch, off):
+    """The short forward copies 16-byte runs of scales: at any other address the call keeps the general
+    kernel's result, plain and (unfused: None) with SwiGLU; the input gradient takes them anywhere."""
+    g = torch.Generator().manual_seed(off)
+    E, N, K = len(HIST), 192, 320
+    rd, n = _routing(dev, HIST)
+    blocks = torch.randint(0, 256, (E, N, K // 32, 16), generator=g, dtype=torch.uint8).to(dev)
+    scales = torch.randint(118, 123, (E, N, K // 32), generator=g, dtype=torch.uint8)
+    store = torch.zeros(scales.numel() + 16, dtype=torch.uint8, device=dev)
+    s = store[off:off + scales.numel()].view(scales.shape)
+    s.copy_(scales)
+    x = torch.randn(n, K, generator=g).to(torch.bfloat16).to(dev)
+    dy = torch.randn(n, N, generator=g).to(torch.bfloat16).to(dev)
+    al = scales.to(dev)
+    y, ref = Q.moe_rows(x, blocks, s, None, rd), Q.moe_rows(x, blocks, al, None, rd)
+    # the same exact products (K of them) in another order of the fp32 sum, then one bf16 rounding each
+    w = Q.mxfp4_to_bf16(blocks, al).float().abs()
+    mag = torch.cat([x[a:a + h].float().abs() @ w[e].t() for e, (a, h) in
+                     enumerate(zip([sum(HIST[:i]) for i in range(E)], HIST))])
+    assert ((y.float() - ref.float()).abs() <= 2 * K * 2.0 ** -24 * mag + 2.0 ** -7 * ref.float().abs()).all()
+    assert Q.moe_rows(x, blocks, s, None, rd, swiglu=("fwd", 1.702, 7.0)) is None
+    monkeypatch.setattr(Q, "DX_SHORT_ROWS", ((1 << 30, 64),))
+    assert torch.equal(Q.moe_rows(dy, blocks, s, None, rd, trans_w=True),
+                       Q.moe_rows(dy, blocks, al, None, rd, trans_w=True))
+
+
 @pytest.mark.parametrize("r", [16, 32])
 @pytest.mark.parametrize("trans_b,K", [(0, 64), (0, 576), (0, 2880), (1, 128), (1, 1472)])
 def test_lora_rows_32_row_map(dev, monkeypatch, r, trans_b, K):
