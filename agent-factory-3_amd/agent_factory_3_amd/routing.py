@@ -184,7 +184,7 @@ class _GateScal(torch.autograd.Function):
 
 def _routing_plan(lg: torch.Tensor, K: int, ei: torch.Tensor | None, ld: int):
     """Routing and its tile metadata in one call (af3_routing_plan): the outputs
-    are slices of one int32 buffer.  Returns (gate_scal, hist, topk_indx,
+    lie in one int32 buffer.  Returns (gate_scal, hist, topk_indx,
     gate_indx, ExptData)."""
     T, E = lg.shape
     R = T * K
@@ -202,6 +202,9 @@ def _routing_plan(lg: torch.Tensor, K: int, ei: torch.Tensor | None, ld: int):
     ws_n = int(lib.af3_routing_plan_workspace_bytes(T, E, K, topk))
     ws = torch.empty(ws_n, dtype=torch.uint8, device=dev) if ws_n else None
     hist, offs, topk_indx, gate_indx, *rest = buf.split(sizes)
+    # tensors of their own to autograd: slices share one version counter, so that an
+    # in-place change of one output would count as a change of those saved for backward
+    hist, offs, topk_indx, gate_indx = hist.data, offs.data, topk_indx.data, gate_indx.data
     _capi.call("af3_routing_plan", lg.data_ptr(), ld, _capi.ptr(ei), topk, T, E, K, gate_scal.data_ptr(),
                hist.data_ptr(), topk_indx.data_ptr(), gate_indx.data_ptr(), offs.data_ptr(),
                (ctypes.c_int32 * nb)(*bms), nb, n_ord, mt, rest[0].data_ptr(), rest[nb].data_ptr(),

@@ -83,6 +83,25 @@ def test_plan_topk_special_logits(dev, T):
     assert torch.equal(R.routing(logits.to(dev), K)[1].src_indx.cpu(), O.routing_topk(logits, K)["topk_indx"])
 
 
+def test_outputs_change_in_place_on_their_own(dev, monkeypatch):
+    """The index tensors share a buffer, not a version: one may change between forward and backward."""
+    monkeypatch.setattr(R, "GAMMA_GRAD", True)
+    g = torch.Generator().manual_seed(3)
+    logits = torch.randn(70, 32, generator=g).to(torch.bfloat16).to(dev)
+    w = torch.randn(280, generator=g).to(torch.bfloat16).to(dev)
+    grads = []
+    for change in (False, True):
+        lg = logits.clone().requires_grad_(True)
+        rd, gi, _ = R.routing(lg, 4)
+        if change:
+            gi.dst_indx.fill_(-1)
+            rd.expt_data.token_offs_raw.zero_()
+            assert [t._version for t in (gi.src_indx, rd.expt_hist)] == [0, 0]
+        rd.gate_scal.backward(w)
+        grads.append(lg.grad)
+    assert torch.equal(grads[0], grads[1]) and grads[0].abs().sum() > 0
+
+
 def test_entry_points_agree(dev):
     """af3_routing_replay / _topk / _replay_noalloc give the plan's outputs."""
     for T, E, K in ((50, 32, 4), (3000, 128, 4)):
