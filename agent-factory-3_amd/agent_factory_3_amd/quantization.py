@@ -1049,12 +1049,14 @@ class Mxfp4Bf16DequantGptOssExperts(nn.Module):
         """The forward-tiled copy of the projection's packed weights
         (``mxfp4_tile_fwd``), made once per weight storage and version (the
         expert weights are frozen); None where the forward cannot read one.
-        ``blocks``: the projection's current uint8 blocks, where the caller has them."""
-        if blocks is None:
+        ``blocks``: the projection's current uint8 blocks, where the caller has
+        them; any that are not the module's storage are not looked at (the
+        cache knows only the module's tensors and their versions)."""
+        src = getattr(self, f"{proj}_blocks", None)
+        if blocks is None or src is None or blocks.data_ptr() != src.data_ptr():
             blocks, _ = self._get_uint8_weights(proj)
         if not blocks.is_cuda or blocks.dim() != 4 or blocks.shape[1] % 32 or blocks.shape[2] % 2:
             return None
-        src = getattr(self, f"{proj}_blocks", None)
         if src is None:
             return None
         cache = self.__dict__.setdefault("_fwd_tiled_cache", {})
@@ -1072,12 +1074,13 @@ class Mxfp4Bf16DequantGptOssExperts(nn.Module):
         """The input gradient's tiled copy of the projection's scales
         (``mxfp4_tile_dx_scales``), made once per scale storage and version;
         None where the input-gradient kernel cannot read one.  ``scales``: the
-        projection's current uint8 scales, where the caller has them."""
-        if scales is None:
+        projection's current uint8 scales, where the caller has them (as in
+        ``_fwd_tiled``)."""
+        src = getattr(self, f"{proj}_scales", None)
+        if scales is None or src is None or scales.data_ptr() != src.data_ptr():
             _, scales = self._get_uint8_weights(proj)
         if not scales.is_cuda or scales.dim() != 3 or scales.shape[1] % 64:
             return None
-        src = getattr(self, f"{proj}_scales", None)
         if src is None:
             return None
         cache = self.__dict__.setdefault("_dx_scales_cache", {})

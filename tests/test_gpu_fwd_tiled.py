@@ -134,6 +134,30 @@ def test_module_cache(dev):
     assert s2 is not s1 and torch.equal(s2, s1)
 
 
+def test_module_copies_follow_the_modules_weights(dev):
+    """With a module the forward multiplies by the module's weights, as the backward does: blocks of another
+    storage, or changed in place, never give the result of a copy made from them earlier."""
+    from agent_factory_3_amd import workloads
+    inp = workloads.layer(2, T=64, E=4, H=256, I=128)
+    m = workloads.make_experts(inp, dev)
+    blocks, scales = m._get_uint8_weights("gate_up_proj")
+    rd, gi, _ = R.routing_replay(inp.logits.to(dev), inp.expt_indx.to(dev), inp.k)
+    x = inp.x.to(dev)
+
+    def fwd(b):
+        return Q.DequantMoEMatmul.apply(x, b, scales, None, rd, gi, None, None, None, None, None, "bf16", inp.k, m,
+                                        "gate_up_proj")
+    want = fwd(blocks)
+    other = blocks.clone().bitwise_not_()
+    assert torch.equal(fwd(other), want)
+    other.copy_(blocks.roll(1, 0))
+    assert torch.equal(fwd(other), want)
+    assert torch.equal(fwd(blocks), want)
+    other = scales + 1
+    ts = m._dx_tiled_scales("gate_up_proj", scales)
+    assert m._dx_tiled_scales("gate_up_proj", other) is ts
+
+
 # rows per expert whose last 128-row tile has 2, 3, 1, 1, 4 and 4 live 32-row
 # groups (tails of 60, 74, 20, 10, 100 and 104 rows) and an idle expert
 COUNTS_NB3 = [700, 330, 660, 650, 100, 360, 0]
