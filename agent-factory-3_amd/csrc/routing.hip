@@ -24,8 +24,8 @@
 //
 // Up to 1024 experts the whole chain (ids and weights, sort, tile maps, work
 // orders) is one launch of one block for small batches and three launches
-// otherwise: every step is a few microseconds of latency, so what a call costs
-// is the number of dependent steps, not bytes.  More experts take the older
+// otherwise: every step is a few microseconds of latency, so what a call
+// costs is the number of dependent steps, not bytes.  More experts take the older
 // chain of one kernel per step.
 #include <mutex>
 
@@ -226,17 +226,15 @@ __global__ void fill_tail_kernel(const int32_t* __restrict__ offs, int E, int64_
 // What bounds it is a chain of short dependent steps, so the steps are merged:
 //   * plan_small_kernel (T K <= 4096 entries): one block does everything;
 //   * larger batches: token_hist_kernel (ids, weights, per-chunk histograms of
-//     64 tokens), plan_scan_kernel (one block: prefix over chunks and experts,
-//     tile maps, work orders), plan_scatter_kernel (stable scatter).
+//     64 to 256 tokens), plan_scan_kernel (one block: prefix over chunks and
+//     experts, tile maps, work orders), plan_scatter_kernel (stable scatter).
 // A token's 16 lanes hold its E logits (E <= 256) and pick the top K by K
 // max-reductions of (order-preserving logit bits, inverted id) keys, so ties
 // go to the lower id; one thread per token with a sorted insertion took
 // 25-45 us (a serial pass over E with one wave per CU).  The rank of an entry
 // among equal ids of its wave comes from ballots over the id's bits instead of
-// a scan of the chunk.  Measured (4 of E, kernel time per call, from ids and
-// weights to the tile maps and work order): top-k of 23 tokens over 32
-// experts 55 -> 10 us, 4096 tokens 79 -> 26 us, replay of 1021 tokens over 128
-// experts 36 -> 24 us, 16384 tokens 52 -> 33 us.
+// a scan of the chunk.  Partial tiles are put in order by a counting sort of
+// their sizes (comparing all pairs of experts took 540 us at 1024).
 // ---------------------------------------------------------------------------
 constexpr int kPlanMaxE = 1024;       // experts (one thread each in the scans)
 constexpr int kPlanMaxTopkE = 256;    // experts of the 16-lane top-k (16 logits per lane)
@@ -245,6 +243,7 @@ constexpr int kPlanSmallTopkT = 256;  // tokens whose top-k the one-block plan t
 constexpr int kPlanSmallCnt = 16384;  // (64-entry group, expert) counters of the one-block plan (64 KB)
 constexpr int kPlanTokens = 64;       // tokens of one pass of 16-lane groups (three-launch plan)
 constexpr int kPlanMaxBm = 8;
+constexpr int kPlanTails = 512;       // sizes of partial tiles sorted at a time
 
 // tile maps and work orders to make (n_bm = 0: none); orders for the first n_order sizes
 struct PlanMaps {
@@ -343,71 +342,116 @@ __device__ __forceinline__ int plan_wave_rank(int e, int ebits, int& count) {
   return __popcll(m & ((1ull << lane) - 1ull));
 }
 
-// inclusive prefix over a wave
+// inclusive prefix over a wave, all lanes active: within rows of 16 lanes, then the
+// last lane of rows 0 and 2 into the next row, then lane 31 into the upper half
+// (a step is one instruction; six shuffles through the LDS unit took ten times it)
 __device__ __forceinline__ int plan_wave_scan(int v) {
-  const int lane = threadIdx.x & 63;
-#pragma unroll
-  for (int o = 1; o < 64; o <<= 1) {
-    const int u = __shfl_up(v, o, 64);
-    if (lane >= o) v += u;
-  }
+  v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);  // row_shr:1
+  v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+  v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);  // row_bcast:15
+  v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);  // row_bcast:31
   return v;
+}
+// the last lane's value
+__device__ __forceinline__ int plan_wave_last(int v) { return __builtin_amdgcn_readlane(v, 63); }
+
+__device__ __forceinline__ int plan_wave_sum(int v) { return plan_wave_last(plan_wave_scan(v)); }
+
+// order j's partial tiles, after the full ones, by decreasing rows (ties to the
+// lower expert): a counting sort of the tails by one wave, kPlanTails sizes at a
+// time from the largest (cnt: LDS), then the -1 padding
+__device__ void plan_tail_order(const PlanMaps& m, int j, int E, const int32_t* counts, int32_t* cnt) {
+  const int lane = threadIdx.x & 63, bm = m.bm[j];
+  int32_t* const out = m.order + (int64_t)j * m.max_tiles;
+  int at = 0;
+  for (int e = lane; e < E; e += 64) at += counts[e] / bm;
+  at = plan_wave_sum(at);  // full tiles
+  const auto sync = [] {  // orders the wave's LDS accesses
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+  };
+  for (int hi = bm; hi > 1; hi -= kPlanTails) {  // tails in [lo, hi), keys hi - 1 - tail
+    const int lo = max(hi - kPlanTails, 1), n_keys = hi - lo;
+    const int bits = n_keys > 1 ? 32 - __clz(n_keys - 1) : 1;
+    for (int i = lane; i < n_keys; i += 64) cnt[i] = 0;
+    sync();
+    for (int e = lane; e < E; e += 64) {
+      const int tail = counts[e] % bm;
+      if (tail >= lo && tail < hi) atomicAdd(&cnt[hi - 1 - tail], 1);
+    }
+    sync();
+    for (int i0 = 0; i0 < n_keys; i0 += 64) {
+      const int v = i0 + lane < n_keys ? cnt[i0 + lane] : 0;
+      const int incl = plan_wave_scan(v);
+      if (i0 + lane < n_keys) cnt[i0 + lane] = at + incl - v;
+      at += plan_wave_last(incl);
+    }
+    sync();
+    for (int e0 = 0; e0 < E; e0 += 64) {
+      const int e = e0 + lane, h = e < E ? counts[e] : 0;
+      const int full = h / bm, tail = h - full * bm;
+      const int key = tail >= lo && tail < hi ? hi - 1 - tail : -1;
+      int c;
+      const int rank = plan_wave_rank(key, bits, c);
+      const int pos = key >= 0 ? cnt[key] + rank : m.max_tiles;
+      if (pos < m.max_tiles) out[pos] = (full << 16) | e;
+      sync();
+      if (key >= 0 && rank == 0) cnt[key] += c;
+      sync();
+    }
+  }
+  for (int i = at + lane; i < m.max_tiles; i += 64) out[i] = -1;
 }
 
 // padded offsets, tile maps and work orders from the experts' counts (LDS, E
-// ints, published by a barrier).  A block of one CU issues one wave
-// instruction per SIMD and cycle, so work that 128 experts need once is not
-// spread over 16 waves that all run it: wave j makes the tile map of size j,
-// wave n_bm + j the order of size j (the whole block scanning one size after
-// another made plan_scan_kernel 22 us at 4096 tokens of 32 experts, this 14).
-__device__ void plan_maps(const PlanMaps& m, int E, const int32_t* counts) {
+// ints, published by a barrier).  A block of one CU issues one wave instruction
+// per SIMD and cycle, so nothing is run by 16 waves that one needs once: a wave
+// makes one order's partial tiles, or the (full) tiles of one map or order for as
+// large a part of the experts as leaves every wave a job.
+__device__ void plan_maps(const PlanMaps& m, int E, const int32_t* counts, int32_t* tails) {
   const int lane = threadIdx.x & 63;
-  const int job = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  if (job >= m.n_bm + m.n_order) return;
-  const bool ord = job >= m.n_bm;
-  const int b = ord ? job - m.n_bm : job;
-  const int bm = m.bm[b];
-  int32_t* const out = (ord ? m.order : m.map) + (int64_t)b * m.max_tiles;
-  int carry = 0;
-  for (int e0 = 0; e0 < E; e0 += 64) {  // (full) tiles in expert order
-    const int e = e0 + lane, h = e < E ? counts[e] : 0;
-    const int n = ord ? h / bm : (h + bm - 1) / bm;
-    const int incl = plan_wave_scan(n), at = carry + incl - n;
-    if (!ord && e < E) m.offs_pad[b * (E + 1) + e] = at;
-    // an expert's first two tiles by its lane, the rest by the wave
-#pragma unroll
-    for (int i = 0; i < 2; ++i)
-      if (i < n && at + i < m.max_tiles) out[at + i] = (i << 16) | e;
-    for (uint64_t big = __ballot(n > 2); big; big &= big - 1) {
-      const int l = __ffsll((unsigned long long)big) - 1;
-      const int n_l = __shfl(n, l, 64), at_l = __shfl(at, l, 64);
-      for (int i = 2 + lane; i < n_l; i += 64)
-        if (at_l + i < m.max_tiles) out[at_l + i] = (i << 16) | (e0 + l);
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int n_grp = (E + 63) >> 6, n_out = m.n_bm + m.n_order;
+  if (n_out == 0) return;
+  if (wave < m.n_order) plan_tail_order(m, wave, E, counts, tails + wave * kPlanTails);
+  const int parts = min(max((16 - m.n_order) / n_out, 1), n_grp), per = (n_grp + parts - 1) / parts;
+  const int first = wave < m.n_order ? wave + 16 : wave;  // (more jobs than waves: n_out > 8)
+  for (int job = first - m.n_order; job < n_out * parts; job += 16) {
+    const int which = job / parts, part = job % parts;
+    const bool ord = which >= m.n_bm;
+    const int b = ord ? which - m.n_bm : which;
+    const int bm = m.bm[b], up = ord ? 0 : bm - 1;
+    int32_t* const out = (ord ? m.order : m.map) + (int64_t)b * m.max_tiles;
+    const int g_end = min(n_grp, (part + 1) * per);
+    int base = 0;  // tiles of the experts before the group
+    if (part > 0) {
+      for (int f = lane; f < min(64 * part * per, E); f += 64) base += (counts[f] + up) / bm;
+      base = plan_wave_sum(base);
     }
-    carry += __shfl(incl, 63, 64);
-  }
-  if (!ord && lane == 0) m.offs_pad[b * (E + 1) + E] = carry;
-  if (ord) {  // then the partial tiles by decreasing rows, ties to the lower expert
-    int n_part = 0;
-    for (int e0 = 0; e0 < E; e0 += 64) {
-      const int e = e0 + lane, h = e < E ? counts[e] : 0;
-      const int full = h / bm, mine = h - full * bm;
-      int rank = 0;
-      for (int f0 = 0; f0 < E; f0 += 64) {  // 64 experts' tails at a time, one per lane
-        const int hf = f0 + lane < E ? counts[f0 + lane] : 0;
-        const int tail = hf % bm;
-        if (e0 == 0) n_part += __popcll(__ballot(tail != 0));
-#pragma unroll 8
-        for (int l = 0; l < 64; ++l) {
-          const int x = __builtin_amdgcn_readlane(tail, l);
-          rank += x > mine || (x == mine && f0 + l < e);
-        }
+    for (int grp = part * per; grp < g_end; ++grp) {
+      const int e = 64 * grp + lane, h = e < E ? counts[e] : 0;
+      const int n = (h + up) / bm;
+      const int incl = plan_wave_scan(n), at = base + incl - n;
+      if (!ord && e < E) m.offs_pad[b * (E + 1) + e] = at;
+      // an expert's first tiles by its lane, the rest by the wave
+      constexpr int kOwn = 8;
+      for (int i = 0; i < kOwn && __ballot(i < n); ++i)
+        if (i < n && at + i < m.max_tiles) out[at + i] = (i << 16) | e;
+      for (uint64_t big = __ballot(n > kOwn); big; big &= big - 1) {
+        const int l = __ffsll((unsigned long long)big) - 1;
+        const int n_l = __shfl(n, l, 64), at_l = __shfl(at, l, 64);
+        for (int i = kOwn + lane; i < n_l; i += 64)
+          if (at_l + i < m.max_tiles) out[at_l + i] = (i << 16) | (64 * grp + l);
       }
-      if (mine && carry + rank < m.max_tiles) out[carry + rank] = (full << 16) | e;
+      base += plan_wave_last(incl);
     }
-    carry += n_part;
+    if (!ord && g_end == n_grp && part * per < n_grp) {  // the part with the last group
+      if (lane == 0) m.offs_pad[b * (E + 1) + E] = base;
+      for (int i = base + lane; i < m.max_tiles; i += 64) out[i] = -1;
+    }
   }
-  for (int i = carry + lane; i < m.max_tiles; i += 64) out[i] = -1;
 }
 
 // hist, offs [E + 1] and start (LDS) = the exclusive prefix of the experts' counts (LDS), by one wave; returns the sum
@@ -423,7 +467,7 @@ __device__ __forceinline__ int plan_offsets(int E, int32_t* counts, int32_t* __r
       offs[e] = carry + incl - h;
       start[e] = carry + incl - h;
     }
-    carry += __shfl(incl, 63, 64);
+    carry += plan_wave_last(incl);
   }
   if (lane == 0) offs[E] = carry;
   return carry;
@@ -445,6 +489,7 @@ __global__ __launch_bounds__(1024) void plan_small_kernel(const uint16_t* __rest
   __shared__ int32_t start[kPlanMaxE];
   __shared__ int32_t counts[kPlanMaxE];
   __shared__ int32_t total;
+  __shared__ int32_t tails[kPlanMaxBm * kPlanTails];
   const int t = threadIdx.x, R = T * K, ngroup = (R + 63) / 64;
   if constexpr (MODE == 2) {
     for (int i = t; i < R; i += 1024) {
@@ -547,7 +592,7 @@ __global__ __launch_bounds__(1024) void plan_small_kernel(const uint16_t* __rest
       gate_scal[i] = 0;
     }
   }
-  plan_maps(m, E, counts);
+  plan_maps(m, E, counts, tails);
 }
 
 // ids and weights (MODE as above) and the expert counts of each chunk of `chunk` tokens: counts[chunk][E]
@@ -589,6 +634,7 @@ __global__ __launch_bounds__(1024) void plan_scan_kernel(int32_t* __restrict__ c
   __shared__ int32_t cnt[kPlanMaxE];
   __shared__ int32_t start[kPlanMaxE];
   __shared__ int32_t seg_sum[1024];
+  __shared__ int32_t tails[kPlanMaxBm * kPlanTails];
   // thread (seg, e): chunks [seg * per, (seg + 1) * per) of expert e
   const int t = threadIdx.x, e = t & (epad - 1), seg = t / epad, nseg = 1024 / epad;
   const int per = (n_chunks + nseg - 1) / nseg;
@@ -627,7 +673,7 @@ __global__ __launch_bounds__(1024) void plan_scan_kernel(int32_t* __restrict__ c
   if (t < E) cnt[t] = all;  // threads 0 .. E - 1 are segment 0
   __syncthreads();
   if (t >= 960) plan_offsets(E, cnt, hist, offs, start);  // the last wave, the maps by the others
-  plan_maps(m, E, cnt);
+  plan_maps(m, E, cnt, tails);
 }
 
 // stable scatter of chunk blockIdx.x into expert-sorted order, and the slots past the valid entries
@@ -869,7 +915,7 @@ static int routing_plan(bool topk, const uint16_t* logits, int64_t ld, const int
     if (rc) return rc;
   }
   const int mode = !topk ? 1 : lane_topk ? 0 : 2;
-  static_assert(kPlanSmallR <= kPlanSmallCnt && 2 * kPlanMaxBm <= 16, "the counters' other use; a wave per map and order");
+  static_assert(kPlanSmallR <= kPlanSmallCnt, "the counters' other use");
   if (plan_one_block(topk, T, E, K)) {
 #define AF3_PLAN(md)                                                                                                 \
   hipLaunchKernelGGL(plan_small_kernel<md>, dim3(1), dim3(1024), 0, stream, logits, ld, expt_indx, (int)T, E, K, ids, \

@@ -46,6 +46,40 @@ def test_plan_matches_oracle(dev, T, E, K, topk):
     _orders(out[0].expt_data, T * K, E)
 
 
+@pytest.mark.parametrize("T,E,K", [(40, 5, 2), (1021, 200, 4), (30000, 70, 4)])
+def test_plan_maps_of_any_block_size(dev, T, E, K):
+    """Maps and orders for every block size the call takes, past the sizes one sorting pass of the tails holds and
+    with experts of many tiles, some of them idle."""
+    g = torch.Generator().manual_seed(E)
+    pref = torch.rand(E, generator=g) ** 6 + 1e-9
+    pref[::3] = 1e-12
+    ids = torch.stack([torch.multinomial(pref, K, replacement=False, generator=g) for _ in range(T)]).to(torch.int32)
+    logits = torch.randn(T, E, generator=g).to(torch.bfloat16)
+    bms = (1, 7, 32, 512, 513, 1300, 3000, 64)
+    lib, ld, idd = _capi.load(), logits.to(dev), ids.to(dev)
+    mt = max(R.max_tiles(T * K, E, bm) for bm in bms)
+    n = int(lib.af3_routing_plan_workspace_bytes(T, E, K, 0))
+    ws = torch.empty(max(n, 1), dtype=torch.uint8, device=dev)
+    hist, topk, gate, offs = (torch.empty(m, dtype=torch.int32, device=dev) for m in (E, T * K, T * K, E + 1))
+    gs = torch.empty(T * K, dtype=torch.bfloat16, device=dev)
+    pad = torch.empty(len(bms), E + 1, dtype=torch.int32, device=dev)
+    maps, orders = (torch.empty(len(bms), mt, dtype=torch.int32, device=dev) for _ in range(2))
+    _capi.call("af3_routing_plan", ld.data_ptr(), E, idd.data_ptr(), 0, T, E, K, gs.data_ptr(), hist.data_ptr(),
+               topk.data_ptr(), gate.data_ptr(), offs.data_ptr(), (ctypes.c_int32 * len(bms))(*bms), len(bms),
+               len(bms), mt, pad.data_ptr(), maps.data_ptr(), orders.data_ptr(), ws.data_ptr(), n,
+               _capi.stream_of(torch.device(dev)))
+    h = torch.bincount(ids.reshape(-1).long(), minlength=E)
+    assert torch.equal(hist.cpu(), h.to(torch.int32))
+    for i, bm in enumerate(bms):
+        want_pad, want_map = O.expt_data(h, bm, mt)
+        assert torch.equal(pad[i].cpu(), want_pad) and torch.equal(maps[i].cpu(), want_map), bm
+        full = [(b << 16) | e for e in range(E) for b in range(int(h[e]) // bm)]
+        tails = sorted([e for e in range(E) if int(h[e]) % bm], key=lambda e: (-(int(h[e]) % bm), e))
+        want = full + [((int(h[e]) // bm) << 16) | e for e in tails]
+        got = orders[i].cpu().tolist()
+        assert got[:len(want)] == want and all(v == -1 for v in got[len(want):]), bm
+
+
 @pytest.mark.parametrize("T", [40, 1100])  # one block, three launches
 def test_plan_drops_out_of_range_ids(dev, T):
     E, K = 12, 4
