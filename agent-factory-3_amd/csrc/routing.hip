@@ -23,8 +23,8 @@
 // shape the reference gives expert-parallel-masked entries.
 //
 // Up to 1024 experts the whole chain (ids and weights, sort, tile maps, work
-// orders) is one launch of one block for small batches and three launches
-// otherwise: every step is a few microseconds of latency, so what a call
+// orders) is one launch of one block for small batches and three or four
+// launches otherwise: every step is a few microseconds of latency, so what a call
 // costs is the number of dependent steps, not bytes.  More experts take the older
 // chain of one kernel per step.
 #include <mutex>
@@ -227,14 +227,22 @@ __global__ void fill_tail_kernel(const int32_t* __restrict__ offs, int E, int64_
 //   * plan_small_kernel (T K <= 4096 entries): one block does everything;
 //   * larger batches: token_hist_kernel (ids, weights, per-chunk histograms of
 //     64 to 256 tokens), plan_scan_kernel (one block: prefix over chunks and
-//     experts, tile maps, work orders), plan_scatter_kernel (stable scatter).
+//     experts, tile maps, work orders), plan_scatter_kernel (stable scatter);
+//   * past kPlanOneScan counts (what the scan's one block holds in registers at a
+//     time) plan_prefix_kernel makes the prefix over the chunks first, 16
+//     experts per block: one block walking the counts in groups of 8 took 70 us
+//     of 92 at 131072 tokens over 128 experts.
 // A token's 16 lanes hold its E logits (E <= 256) and pick the top K by K
 // max-reductions of (order-preserving logit bits, inverted id) keys, so ties
 // go to the lower id; one thread per token with a sorted insertion took
 // 25-45 us (a serial pass over E with one wave per CU).  The rank of an entry
 // among equal ids of its wave comes from ballots over the id's bits instead of
 // a scan of the chunk.  Partial tiles are put in order by a counting sort of
-// their sizes (comparing all pairs of experts took 540 us at 1024).
+// their sizes (comparing all pairs of experts took 540 us at 1024).  Measured (4
+// of E, kernel time per call from ids and weights to the tile maps and work
+// order, against one kernel per step): top-k of 23 tokens over 32 experts 51 ->
+// 6.4 us, 4096 tokens 61 -> 16; replay of 1021 tokens over 128 experts 27 -> 15,
+// 16384 tokens 30 -> 17, 131072 tokens 60 -> 47.
 // ---------------------------------------------------------------------------
 constexpr int kPlanMaxE = 1024;       // experts (one thread each in the scans)
 constexpr int kPlanMaxTopkE = 256;    // experts of the 16-lane top-k (16 logits per lane)
@@ -244,6 +252,9 @@ constexpr int kPlanSmallCnt = 16384;  // (64-entry group, expert) counters of th
 constexpr int kPlanTokens = 64;       // tokens of one pass of 16-lane groups (three-launch plan)
 constexpr int kPlanMaxBm = 8;
 constexpr int kPlanTails = 512;       // sizes of partial tiles sorted at a time
+constexpr int kPlanSeg = 32;          // chunks per thread and round of the prefix over chunks (in registers)
+constexpr int kPlanOneScan = 1024 * kPlanSeg;  // counts up to which plan_scan_kernel takes the prefix along
+constexpr int kPlanPrefixE = 16;      // experts per block of the prefix kernel
 
 // tile maps and work orders to make (n_bm = 0: none); orders for the first n_order sizes
 struct PlanMaps {
@@ -627,53 +638,86 @@ __global__ __launch_bounds__(1024) void token_hist_kernel(const uint16_t* __rest
   for (int e = t; e < E; e += 1024) counts[(int64_t)blockIdx.x * E + e] = sh[e];
 }
 
-// one block: counts[chunk][E] -> exclusive prefix over the chunks (in place), hist, offs, tile maps and orders
+// counts[chunk][e] -> their exclusive prefix over the chunks, in place; returns
+// the sum.  `width` (a power of two) threads side by side take as many experts,
+// the block's 1024 / width segments of them kPlanSeg chunks each: a round's counts
+// are read once, all in flight together, and held for the write.
+__device__ int plan_prefix(int32_t* __restrict__ counts, int n_chunks, int E, int e, int width, int32_t* seg_sum) {
+  const int t = threadIdx.x, x = t & (width - 1), seg = t / width, nseg = 1024 / width;
+  int32_t* const col = counts + min(e, E - 1);
+  int carry = 0;
+  for (int b0 = 0; b0 < n_chunks; b0 += nseg * kPlanSeg) {
+    const int per = min(kPlanSeg, (n_chunks - b0 + nseg - 1) / nseg);
+    const int c0 = b0 + seg * per, n = e < E ? min(per, n_chunks - c0) : 0;  // n < 0: none
+    int u[kPlanSeg];
+#pragma unroll
+    for (int j0 = 0; j0 < kPlanSeg; j0 += 8)
+      if (j0 < per) {
+#pragma unroll
+        for (int j = j0; j < j0 + 8; ++j) u[j] = col[(int64_t)min(c0 + j, n_chunks - 1) * E];
+      }
+    int sum = 0;
+#pragma unroll
+    for (int j0 = 0; j0 < kPlanSeg; j0 += 8)
+      if (j0 < per) {
+#pragma unroll
+        for (int j = j0; j < j0 + 8; ++j) {
+          u[j] = j < n ? u[j] : 0;
+          sum += u[j];
+        }
+      }
+    seg_sum[t] = sum;
+    __syncthreads();
+    int run = carry, all = 0;
+#pragma unroll 4
+    for (int s = 0; s < nseg; ++s) {
+      const int v = seg_sum[s * width + x];
+      run += s < seg ? v : 0;
+      all += v;
+    }
+#pragma unroll
+    for (int j0 = 0; j0 < kPlanSeg; j0 += 8)
+      if (j0 < per) {
+#pragma unroll
+        for (int j = j0; j < j0 + 8; ++j) {
+          if (j < n) col[(int64_t)(c0 + j) * E] = run;
+          run += u[j];
+        }
+      }
+    carry += all;
+    __syncthreads();
+  }
+  return carry;
+}
+
+// the prefix over the chunks of kPlanPrefixE experts per block, and hist
+__global__ __launch_bounds__(1024) void plan_prefix_kernel(int32_t* __restrict__ counts, int n_chunks, int E,
+                                                           int32_t* __restrict__ hist) {
+  __shared__ int32_t seg_sum[1024];
+  const int t = threadIdx.x, e = blockIdx.x * kPlanPrefixE + (t & (kPlanPrefixE - 1));
+  const int all = plan_prefix(counts, n_chunks, E, e, kPlanPrefixE, seg_sum);
+  if (t < kPlanPrefixE && e < E) hist[e] = all;
+}
+
+// one block: counts[chunk][E] -> exclusive prefix over the chunks (n_chunks 0:
+// done, hist holds the sums), then hist, offs, tile maps and orders
 __global__ __launch_bounds__(1024) void plan_scan_kernel(int32_t* __restrict__ counts, int n_chunks, int E, int epad,
                                                          int32_t* __restrict__ hist, int32_t* __restrict__ offs,
                                                          PlanMaps m) {
   __shared__ int32_t cnt[kPlanMaxE];
   __shared__ int32_t start[kPlanMaxE];
-  __shared__ int32_t seg_sum[1024];
-  __shared__ int32_t tails[kPlanMaxBm * kPlanTails];
-  // thread (seg, e): chunks [seg * per, (seg + 1) * per) of expert e
-  const int t = threadIdx.x, e = t & (epad - 1), seg = t / epad, nseg = 1024 / epad;
-  const int per = (n_chunks + nseg - 1) / nseg;
-  const int c0 = min(seg * per, n_chunks), c1 = e < E ? min(c0 + per, n_chunks) : c0;
-  auto load8 = [&](int c, int (&u)[8]) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) u[j] = counts[(int64_t)min(c + j, c1 - 1) * E + e];
-#pragma unroll
-    for (int j = 0; j < 8; ++j) u[j] = c + j < c1 ? u[j] : 0;
-  };
-  int sum = 0;
-  for (int c = c0; c < c1; c += 8) {
-    int u[8];
-    load8(c, u);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) sum += u[j];
+  __shared__ int32_t scratch[kPlanMaxBm * kPlanTails];
+  static_assert(kPlanMaxBm * kPlanTails >= 1024, "the segments' sums, then the tails");
+  const int t = threadIdx.x;
+  if (n_chunks > 0) {
+    const int all = plan_prefix(counts, n_chunks, E, t & (epad - 1), epad, scratch);
+    if (t < E) cnt[t] = all;  // threads 0 .. E - 1 are segment 0
+  } else if (t < E) {
+    cnt[t] = hist[t];
   }
-  seg_sum[t] = sum;
-  __syncthreads();
-  int run = 0, all = 0;
-#pragma unroll 4
-  for (int s = 0; s < nseg; ++s) {
-    const int x = seg_sum[s * epad + e];
-    run += s < seg ? x : 0;
-    all += x;
-  }
-  for (int c = c0; c < c1; c += 8) {
-    int u[8];
-    load8(c, u);
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      if (c + j < c1) counts[(int64_t)(c + j) * E + e] = run;
-      run += u[j];
-    }
-  }
-  if (t < E) cnt[t] = all;  // threads 0 .. E - 1 are segment 0
   __syncthreads();
   if (t >= 960) plan_offsets(E, cnt, hist, offs, start);  // the last wave, the maps by the others
-  plan_maps(m, E, cnt, tails);
+  plan_maps(m, E, cnt, scratch);
 }
 
 // stable scatter of chunk blockIdx.x into expert-sorted order, and the slots past the valid entries
@@ -937,8 +981,15 @@ static int routing_plan(bool topk, const uint16_t* logits, int64_t ld, const int
   int rc = af3::check_launch("routing/token_hist");
   if (rc) return rc;
   const int epad = 1 << ebits;  // >= E, <= 1024
-  hipLaunchKernelGGL(plan_scan_kernel, dim3(1), dim3(1024), 0, stream, counts, n_chunks, E, epad, hist, token_offs_raw,
-                     m);
+  const bool one_scan = lay.rows * epad <= kPlanOneScan;
+  if (!one_scan) {
+    hipLaunchKernelGGL(plan_prefix_kernel, dim3((unsigned)af3_cdiv(E, kPlanPrefixE)), dim3(1024), 0, stream, counts,
+                       n_chunks, E, hist);
+    rc = af3::check_launch("routing/prefix");
+    if (rc) return rc;
+  }
+  hipLaunchKernelGGL(plan_scan_kernel, dim3(1), dim3(1024), 0, stream, counts, one_scan ? n_chunks : 0, E, epad, hist,
+                     token_offs_raw, m);
   rc = af3::check_launch("routing/scan");
   if (rc) return rc;
   hipLaunchKernelGGL(plan_scatter_kernel, dim3(n_chunks), dim3(256), 0, stream, ids, scal, R, E,

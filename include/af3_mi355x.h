@@ -100,7 +100,7 @@ int af3_routing_topk(const uint16_t* logits, int64_t ld_logits, int64_t n_tokens
 /* Routing (topk != 0: af3_routing_topk, else af3_routing_replay) and the tile
  * metadata of its result (af3_expt_data for every size of the host array
  * block_ms, af3_tile_order for the first n_orders of them) in one call: one
- * launch for small batches, three otherwise.  token_offs_pad [n_block_ms][E+1],
+ * launch for small batches, three or four otherwise.  token_offs_pad [n_block_ms][E+1],
  * block_pid_map [n_block_ms][max_tiles], orders [n_orders][max_tiles], all -1
  * past each size's tiles; E <= 1024, n_block_ms <= 8.  The workspace is
  * af3_routing_plan_workspace_bytes (0 for the one-launch form).  No counterpart

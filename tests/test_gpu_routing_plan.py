@@ -46,6 +46,19 @@ def test_plan_matches_oracle(dev, T, E, K, topk):
     _orders(out[0].expt_data, T * K, E)
 
 
+# the prefix over chunks in its own launch: just past the one-block limit, experts past whole blocks of 16, more
+# chunks than a block's segments hold in one round; the most counts the scan kernel takes along
+@pytest.mark.parametrize("T,E,K", [(2049, 1024, 4), (2048, 1024, 4), (16385, 128, 4), (16384, 128, 4), (9000, 250, 1),
+                                   (140000, 17, 4)])
+def test_plan_prefix_over_many_chunks(dev, T, E, K):
+    g = torch.Generator().manual_seed(T + E)
+    logits = torch.randn(T, E, generator=g).to(torch.bfloat16)
+    ids = torch.rand(T, E, generator=g).topk(K, dim=1).indices.to(torch.int32)
+    out, ref = R.routing_replay(logits.to(dev), ids.to(dev), K), O.routing_replay(logits, ids, K)
+    _check(*out, ref)
+    _orders(out[0].expt_data, T * K, E)
+
+
 @pytest.mark.parametrize("T,E,K", [(40, 5, 2), (1021, 200, 4), (30000, 70, 4)])
 def test_plan_maps_of_any_block_size(dev, T, E, K):
     """Maps and orders for every block size the call takes, past the sizes one sorting pass of the tails holds and
