@@ -17,6 +17,13 @@
 // their order, so the logits are unchanged.  Measured: 1
 // row, E 128 36 -> 16 us; 23 rows, E 32 33 -> 14; 4096 rows, E 32 41 -> 18; 1021
 // rows, E 128 48 -> 24; 16384 rows, E 128 53 -> 30 (LDS reads bound it now).
+// Several blocks per CU hide each other's latency, and what the ring's depth costs
+// is blocks per CU: past 256 blocks it has two stages (three at E 65 - 128 and H
+// >= 2048, where the W tile's latency shows), and 129 - 192 experts are padded to
+// 192 columns instead of 256 where the products count (H >= 512).  65536 rows,
+// kernel time, plain double buffer / deep ring / these: H 2880, E 8 64 / 66 / 64,
+// E 128 114 / 104 / 100, E 160 125 / 136 / 116, E 256 167 / 149 / 139; H 512, E 64
+// 15 / 22 / 14, E 128 20 / 27 / 17; H 64, E 128 8.7 / 12.8 / 7.5.
 // LDS chunks of 16 bytes are XOR-swizzled by row (the copy writes LDS linearly,
 // so the lanes' source addresses carry the swizzle).  k is permuted
 // identically on both operands: lane (r, h) of v_mfma_f32_32x32x16_bf16 feeds
@@ -27,14 +34,16 @@ namespace {
 
 constexpr int kRtRows = 64;  // rows per block
 constexpr int kRtBK = 64;    // k per step
+constexpr unsigned kRtOneRound = 256;  // blocks up to which the deep rings are taken (one per CU)
 
 // one 16-byte global -> LDS copy per lane (LDS address: wave-uniform base + 16 lane)
 __device__ __forceinline__ void rt_dma16(const void* gptr, uint32_t lds_byte_addr) {
   asm volatile("s_nop 0\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(gptr), "{m0}"(lds_byte_addr) : "memory");
 }
 
-// EP columns computed (E rounded up to 32, 64, 128 or 256), TW 32-column tiles per wave, ST ring stages
-template <int EP, int TW, int ST>
+// EP columns computed (E rounded up to 32, 64, 128, 192 or 256), TW 32-column tiles per wave, ST ring stages
+// (ONCE: no k-step is copied twice, two stages only)
+template <int EP, int TW, int ST, bool ONCE = false>
 __global__ __launch_bounds__(EP / TW * 4) void router_kernel(const uint16_t* __restrict__ x, int64_t ldx,
                                                              const uint16_t* __restrict__ w, int64_t ldw,
                                                              const uint16_t* __restrict__ bias, int64_t T, int H, int E,
@@ -66,8 +75,11 @@ __global__ __launch_bounds__(EP / TW * 4) void router_kernel(const uint16_t* __r
   }
   const uint32_t lds0 = __builtin_amdgcn_readfirstlane(
       (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)lds);
-  // k-steps past the end copy the last one again, into a stage no wave reads again
+  // k-steps past the end copy the last one again, into a stage no wave reads again (no branch
+  // in the loop), unless there are so few that this counts
+  static_assert(!ONCE || ST == 2, "the wait counts the repeated copies");
   auto issue = [&](int kk) {
+    if (ONCE && kk >= nk) return;
     const int ks = min(kk, nk - 1);
     const uint32_t st = lds0 + (uint32_t)((kk % ST) * STAGE + wave * CPW * 1024);
 #pragma unroll
@@ -119,6 +131,11 @@ __global__ __launch_bounds__(EP / TW * 4) void router_kernel(const uint16_t* __r
   }
 }
 
+template <int EP, int TW, int ST, bool ONCE = false>
+constexpr unsigned router_threads() {
+  return EP / TW * 4;
+}
+
 }  // namespace
 
 extern "C" int af3_router_logits(const uint16_t* x, int64_t ldx, const uint16_t* w, int64_t ldw, const uint16_t* bias,
@@ -134,17 +151,35 @@ extern "C" int af3_router_logits(const uint16_t* x, int64_t ldx, const uint16_t*
   if (n_tokens == 0) return 0;
   AF3_REQUIRE(x && w && logits, "router_logits: null pointer");
   const dim3 grid((unsigned)af3_cdiv(n_tokens, kRtRows));
-#define AF3_RT(ep, tw, st)                                                                                        \
-  hipLaunchKernelGGL((router_kernel<ep, tw, st>), grid, dim3(ep / tw * 4), 0, stream, x, ldx, w, ldw, bias, n_tokens, \
-                     hidden, n_expts, logits, ld_logits)
-  if (n_expts <= 32)
-    AF3_RT(32, 1, 6);   // 12 KB stages, 6 copies per wave and step
-  else if (n_expts <= 64)
-    AF3_RT(64, 1, 8);   // 16 KB, 4
-  else if (n_expts <= 128)
-    AF3_RT(128, 1, 6);  // 24 KB, 3
-  else
-    AF3_RT(256, 2, 4);  // 40 KB, 5
+#define AF3_RT(...)                                                                                               \
+  hipLaunchKernelGGL((router_kernel<__VA_ARGS__>), grid, dim3(router_threads<__VA_ARGS__>()), 0, stream, x, ldx, w, \
+                     ldw, bias, n_tokens, hidden, n_expts, logits, ld_logits)
+  const bool once = hidden <= 128;  // one or two k-steps: a repeated copy counts
+  if (grid.x <= kRtOneRound) {
+    if (n_expts <= 32)
+      AF3_RT(32, 1, 6);   // 12 KB stages, 6 copies per wave and step
+    else if (n_expts <= 64)
+      AF3_RT(64, 1, 8);   // 16 KB, 4
+    else if (n_expts <= 128)
+      AF3_RT(128, 1, 6);  // 24 KB, 3
+    else
+      AF3_RT(256, 2, 4);  // 40 KB, 5
+  } else if (n_expts <= 32) {
+    if (once) AF3_RT(32, 1, 2, true);
+    else AF3_RT(32, 1, 2);
+  } else if (n_expts <= 64) {
+    if (once) AF3_RT(64, 1, 2, true);
+    else AF3_RT(64, 1, 2);
+  } else if (n_expts <= 128) {
+    if (once) AF3_RT(128, 1, 2, true);
+    else if (hidden < 2048) AF3_RT(128, 1, 2);
+    else AF3_RT(128, 1, 3);
+  } else if (n_expts <= 192 && hidden >= 512) {
+    AF3_RT(192, 3, 2);    // 32 KB, 8
+  } else {
+    if (once) AF3_RT(256, 2, 2, true);
+    else AF3_RT(256, 2, 2);
+  }
 #undef AF3_RT
   return af3::check_launch("router_logits");
 }

@@ -215,3 +215,18 @@ def test_router_ring_edges(dev, T, H, E):
     got = R.router_logits_hip(x.to(dev), w.to(dev), None)
     ref, mag = O.router_logits(x, w, None)
     check_close(got, ref, mag=mag, n=H, what=f"router T={T} H={H} E={E}")
+
+
+@pytest.mark.parametrize("H", [64, 128, 192, 512, 2048])
+@pytest.mark.parametrize("E", [8, 33, 128, 160, 193, 256])
+def test_router_past_one_block_per_cu(dev, H, E):
+    """More than 256 blocks take two or three stages and other column paddings: the same sums, so the logits of
+    the first 256 blocks are those of a smaller batch, bit for bit."""
+    T = 256 * 64 + 65
+    g = torch.Generator().manual_seed(H + E)
+    x = torch.randn(T, H, generator=g).to(torch.bfloat16).to(dev)
+    w = (torch.randn(E, H, generator=g) * H ** -0.5).to(torch.bfloat16).to(dev)
+    b = torch.randn(E, generator=g).to(torch.bfloat16).to(dev)
+    got = R.router_logits_hip(x, w, b)
+    assert torch.equal(got[:16384], R.router_logits_hip(x[:16384], w, b))
+    assert torch.equal(got[16000:], R.router_logits_hip(x[16000:], w, b))
