@@ -61,25 +61,31 @@ GEMM_BLOCK_M = 128
 # explicitly selected configurations, and the C library's tile_cfg (0 =
 # default).  The default kernels take the map of fwd_block_m (forward, tile_cfg
 # 26) and dx_block_m (input gradient, tile_cfg 28), both 128; 256 there selects
-# the 256 x 256 kernels (tile_cfg 22 / 23).  The LoRA row products always use
-# the 128-row map.  x_off32: tell the library when x lies within 4 GiB (the
+# the 256 x 256 kernels (tile_cfg 22 / 23).  x_off32: tell the library when x lies within 4 GiB (the
 # forward then addresses it by a scalar base and 32-bit offsets).
 # With few rows per expert (routed rows <= the limit times the experts) they take
 # the 32- or 64-row map and the short-tile kernels (tile_cfg 27 / 29) instead.
-# Measured, both launches of a 120b layer (E 128, top-4, rank 32), us, 128- /
-# 32- / 64-row map: forward 301 tokens (9 rows per expert) 409 / 354 / 361, 600
-# (19) 421 / 373 / 377, 1021 (32) 460 / 537 / 422, 1500 (47) 488 / 731 / 465,
-# under Zipf loads 600 441 / 404 / 408, 1500 551 / 562 / 531; input gradient 40
-# (1) 345 / 294 / 338, 301 420 / 382 / 398, 600 437 / 400 / 416, 1021 467 / 601 /
-# 449, 1500 513 / 993 / 620, Zipf 400 438 / 422 / 446, 600 454 / 491 / 470, 1021
-# 555 / 552 / 527.
+# Measured, both launches of a layer at these rows per expert, us, 128- / 32- /
+# 64-row map.  Forward, 128 experts, rank 32: 8 rows 397 / 336 / 348, 19 417 / 363 /
+# 370, 24 424 / 397 / 381, 32 449 / 530 / 409, 48 488 / 734 / 467, 56 499 / 731 / 493;
+# Zipf loads 19 441 / 407 / 402, 32 510 / 470 / 454, 48 539 / 572 / 539; 32 experts: 8
+# 124 / 98 / 109, 24 131 / 110 / 116, 48 149 / 163 / 128, 64 153 / 193 / 186.  Input
+# gradient, 128 experts: 1 264 / 247 / 238, 8 403 / 365 / 386, 16 418 / 382 / 396, 19 425
+# / 387 / 403, 24 435 / 442 / 415, 32 463 / 582 / 448, 40 501 / 743 / 498; 32 experts: 8
+# 125 / 113 / 117, 19 130 / 120 / 123, 32 147 / 170 / 142, 48 156 / 185 / 151.  Under
+# Zipf loads (the fuller experts' tiles then start another round of blocks) the
+# gradient gains 4-6% up to 12 rows (32) and 2-6% from 22 to 32 (64); between them it
+# is within 3% of the 128-row map either way (13-18 rows on 32: 0 to -3%, where the
+# 64-row map is 2-5% behind; 19-21 on 64: 0 to -3%, on 32 -5 to -7%), while even
+# loads gain 5-11% there.  Loads on a few experts only (4 or 16 of 128) lose up to 10%
+# forward and 30% in the gradient past 10 rows; the loads are not known on the host.
 GEMM_TILE = {"block_m": 256, "tile_cfg": 0, "fwd_block_m": 128, "dx_block_m": 128, "short": True}
 FWD_SHORT_ROWS = ((24, 32), (48, 64))   # (rows per expert at most, block_m)
+DX_SHORT_ROWS = ((18, 32), (32, 64))
 # LoRA row products take the 32-row map while its tiles are resident at once (two
 # blocks of 64 KB LDS on each of 256 CUs): the two launches at 2000 tokens over 128
 # experts (378 tiles) 86 -> 54 us, at 4096 (640 tiles) 86 against 89.
 LORA_SHORT_TILES = 512
-DX_SHORT_ROWS = ((13, 32), (32, 64))
 
 # The expert module's forward GEMMs read a tiled copy of each frozen
 # projection's packed weights (af3_mxfp4_tile_fwd: the words one k-step of a

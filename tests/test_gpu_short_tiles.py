@@ -124,6 +124,14 @@ def test_map_choice(dev):
     assert 32 not in big.block_pid_map and Q._short_block_m(big, 100, 16, 5760, 2880, False, True) == 0
 
 
+@pytest.mark.parametrize("trans,rows,want", [(False, 24, 32), (False, 25, 64), (False, 48, 64), (False, 49, 0),
+                                             (True, 18, 32), (True, 19, 64), (True, 32, 64), (True, 33, 0)])
+def test_map_choice_at_its_lines(trans, rows, want):
+    ed = R.ExptData(None, None, block_pid_map={32: 0, 64: 0}, gemm_order={32: 0, 64: 0})
+    for E in (32, 128):
+        assert Q._short_block_m(ed, rows * E, E, 2880, 2880, trans, True) == want
+
+
 @pytest.mark.parametrize("off", [1, 8])
 def test_scales_at_an_unaligned_address(dev, monkeypatch, off):
     """The short forward copies 16-byte runs of scales: at any other address the call keeps the general
