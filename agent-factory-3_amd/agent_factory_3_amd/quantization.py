@@ -52,7 +52,7 @@ from torch import nn
 from . import _capi, kernels
 from .kernels import mxfp4_to_bf16_hip, swiglu_backward_raw, swiglu_forward
 from .routing import (  # noqa: F401  (re-exported names of the routing layer)
-    ExptData, GatherIndx, RoutingData, ScatterIndx, compute_expt_data, compute_expt_data_torch,
+    SHORT_TILES, ExptData, GatherIndx, RoutingData, ScatterIndx, compute_expt_data, compute_expt_data_torch,
     dense_routing, gemm_order_for, max_tiles, router_linear, routing, routing_replay,
 )
 
@@ -85,7 +85,7 @@ DX_SHORT_ROWS = ((18, 32), (32, 64))
 # LoRA row products take the 32-row map while its tiles are resident at once (two
 # blocks of 64 KB LDS on each of 256 CUs): the two launches at 2000 tokens over 128
 # experts (378 tiles) 86 -> 54 us, at 4096 (640 tiles) 86 against 89.
-LORA_SHORT_TILES = 512
+LORA_SHORT_TILES = SHORT_TILES
 
 # The expert module's forward GEMMs read a tiled copy of each frozen
 # projection's packed weights (af3_mxfp4_tile_fwd: the words one k-step of a

@@ -31,7 +31,7 @@ GEMM_ORDER_BMS = (128,)  # tile sizes whose full-first work order is made with t
 # default GEMMs and the LoRA row tiles); other sizes get theirs on first use (gemm_order_for)
 SHORT_BLOCK_MS = (32, 64)  # tile sizes of the short-tile GEMMs, mapped where the rows are few per expert
 SHORT_ROWS_PER_EXPERT = 64  # (routed rows <= this many per expert, or at most SHORT_TILES 32-row tiles)
-SHORT_TILES = 512
+SHORT_TILES = 512           # (the LoRA row products' limit: quantization.LORA_SHORT_TILES)
 PLAN_MAX_E = 1024  # experts of af3_routing_plan (routing and tile metadata in one call)
 
 

@@ -211,7 +211,7 @@ __global__ __launch_bounds__(256, 6) void lora_merge_generic_kernel(const uint8_
 // tile is computed.
 // HBM bounds it, and the reads cost more than their share: 32 experts' gate_up at
 // r 16 take 159 us [E][K][N] / 112 us [E][N][K] without the stores, and 251 / 200
-// us with loads that all hit in L2, where the whole takes 358 / 331.  So a unit
+// us with loads that all hit in L2, where the whole takes 362 / 337.  So a unit
 // reads 128 bytes of each packed row (a whole line; 64 bytes per unit: 387 / 343
 // us, codes loaded non-temporally: 517 / 344), and units are dealt to the XCDs
 // in contiguous runs (k-tile fastest), so the blocks that share lines of packed
@@ -219,8 +219,8 @@ __global__ __launch_bounds__(256, 6) void lora_merge_generic_kernel(const uint8_
 // r 16 but no better at r 32.  Two to six tiles of loads in flight changed
 // nothing.  Against the form before (64 x 64 tiles by four waves together, the
 // delta as fp32 and the sum as bf16 through LDS, three block barriers per tile):
-// r 16 377 / 368 -> 358 / 331 us, r 32 411 / 404 -> 395 / 358 (1.36 GB, 3.8 / 4.1
-// TB/s).
+// r 16 377 / 370 -> 362 / 337 us (1.36 GB, 3.7 / 4.0 TB/s), r 32 411 / 405 -> 409 /
+// 352, r 64 538 / 532 -> 525 / 447.
 constexpr int kMgWaves = 8;     // waves of a block
 constexpr int kMgBK = 32 * kMgWaves;  // k columns of a unit
 constexpr int kMgRun = 8;       // n-tiles of a unit (fewer where the launch has few units)
@@ -406,10 +406,7 @@ extern "C" int af3_mxfp4_lora_merge(const uint8_t* blocks, const uint8_t* scales
   AF3_REQUIRE(((uintptr_t)blocks & 3) == 0 && ((uintptr_t)lora_b & 15) == 0 && ((uintptr_t)lora_a & 15) == 0 &&
                   ((uintptr_t)out & 15) == 0,
               "mxfp4_lora_merge: blocks must be 4-byte, lora_a, lora_b and out 16-byte aligned");
-  const int ntn = (int)af3_cdiv(N, kMgN), ntk = (int)af3_cdiv(K, kMgK);
-  const int64_t tiles = (int64_t)E * ntn * ntk;
-  const int64_t per_xcd = af3_cdiv(tiles, 8);
-  // resident blocks per XCD: 32 CUs x 6 blocks of 26 KB LDS
+  const int ntn = (int)af3_cdiv(N, kMgN);
   if (r <= 64) {
     const int nk = (int)af3_cdiv(K, kMgBK);
     int run = kMgRun;  // shorter runs while the launch would leave CUs idle
@@ -433,6 +430,10 @@ extern "C" int af3_mxfp4_lora_merge(const uint8_t* blocks, const uint8_t* scales
 #undef AF3_MGR
 #undef AF3_MG
   } else {
+    const int ntk = (int)af3_cdiv(K, kMgK);
+    const int64_t tiles = (int64_t)E * ntn * ntk;
+    const int64_t per_xcd = af3_cdiv(tiles, 8);
+    // resident blocks per XCD: 32 CUs x 6 blocks of 26 KB LDS
     const int bpx = (int)(per_xcd < kMgBlocksPerXcd ? per_xcd : kMgBlocksPerXcd);
     hipLaunchKernelGGL(lora_merge_generic_kernel, dim3((unsigned)(8 * bpx)), dim3(256), 0, stream, blocks, scales,
                        lora_a, lora_b, scaling, out, N, K, r, layout, ntn, ntk, tiles, per_xcd, bpx);

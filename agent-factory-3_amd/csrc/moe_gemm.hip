@@ -624,7 +624,10 @@ static inline unsigned g4_grid(int max_tiles, int NN, int GM) {
 // Work item of the short-tile kernels (32 / 64-row maps) when there are fewer
 // than kG9SpreadTiles m-tiles: the unit dealt to the XCDs in turn is GM m-tiles
 // x one n-tile.  Dealing whole groups of n-tiles as g4_work_item does would
-// leave XCDs idle then (one token: 4 m-tiles, two groups).
+// leave XCDs idle then (one token: 4 m-tiles, two groups).  Both launches of a
+// forward, rank 32, grouped / spread: 4 m-tiles 44 / 36 us, 8 47 / 39, 12 48 / 48, 16
+// 49 / 49, 20 71 / 56, 24 83 / 82, 32 92 / 92; of an input gradient the same within 2%
+// up to 16, then 20 99 / 87, 24 103 / 108, 32 109 / 124, 64 186 / 228.
 __device__ __forceinline__ bool g9_work_item(const Params& p, int& mt, int& nt) {
   const int NN = p.n_nblk, Mt = p.tile_offs[p.E], GM = p.group_m;
   const int x = blockIdx.x & 7, j = blockIdx.x >> 3;
@@ -2950,7 +2953,7 @@ static int moe_gemm_impl(const uint16_t* x, int64_t ldx, const int32_t* gather_i
   //   4 / 2: gemm2, 256x256 / 128x256 tiles with the weight dequantised into
   //       LDS (general fallback for block_m 256 / 128)
   //   9: single-buffered 128x128 row tiles (any K % 32 == 0; used when K % 64 != 0)
-  //   tile_cfg / 100 = m-tiles per group of the 22 / 23 / 26 - 29 work order (default 4; 2 for 26 / 28)
+  //   tile_cfg / 100 = m-tiles per group of the 22 / 23 / 26 - 29 work order (default 4; 2 for 26 - 29)
   int cfg = tile_cfg % 100;
   const int group_m = tile_cfg / 100 > 0 ? tile_cfg / 100 : 4;
   if (cfg == 0) {

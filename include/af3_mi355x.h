@@ -156,11 +156,11 @@ int af3_tile_order(const int32_t* hist, int n_expts_tot, int block_m, const int3
  * block_m 128 -> 26 (forward, 128 x 256 work items, two blocks per CU) and
  * 28 (input gradient, same shape); block_m 32 / 64 -> 27 / 29, the same k-loops
  * on 32 / 64 x 256 items for few rows per expert (AF3_EUNSUPPORTED, nothing
- * launched, unless AF3_X_OFFSETS_32 is set, N % 64 == 0 and K % 320 == 0 (27; K
- * <= 3072) or K % 64 == 0 (29)); block_m 256 -> 22 / 23 (256 x 256); the
+ * launched, unless AF3_X_OFFSETS_32 is set, N % 64 == 0 and K % 320 == 0 with
+ * 16-byte aligned w_scales (27; K <= 3072) or K % 64 == 0 (29)); block_m 256 -> 22 / 23 (256 x 256); the
  * general fallbacks 4 / 2 / 9 where a default's alignment or K % 64 == 0
  * requirement fails.  tile_cfg / 100 = m-tiles per work group of the
- * 22 / 23 / 26 / 28 order (default 4; 2 for 26 / 28).  tile_cfg |
+ * 22 / 23 / 26 - 29 order (default 4; 2 for 26 - 29).  tile_cfg |
  * AF3_W_FWD_TILED: w_blocks is the af3_mxfp4_tile_fwd copy of the weights
  * (trans_w 0, the tile_cfg 26 / 27 forward only; AF3_EUNSUPPORTED, nothing
  * launched, when another kernel is selected: the caller then passes the
