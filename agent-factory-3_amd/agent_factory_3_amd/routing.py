@@ -194,7 +194,9 @@ def _routing_plan(lg: torch.Tensor, K: int, ei: torch.Tensor | None, ld: int):
     tiles = [max_tiles(R, E, bm) for bm in bms]
     mt = max(tiles)
     n_ord = max(bms.index(bm) for bm in GEMM_ORDER_BMS) + 1   # orders for the leading sizes
-    sizes = [E, E + 1, R, R] + [E + 1] * nb + [mt] * (nb + n_ord)
+    sizes = [E, E + 1, R, R] + [E + 1] * nb + [mt] * nb
+    for n in tiles[:n_ord]:   # an order's slots past its size's most tiles are not handed out
+        sizes += [n, mt - n]
     buf = torch.empty(sum(sizes), dtype=torch.int32, device=dev)
     gate_scal = torch.empty(R, dtype=torch.bfloat16, device=dev)
     lib = _capi.load()
@@ -214,7 +216,7 @@ def _routing_plan(lg: torch.Tensor, K: int, ei: torch.Tensor | None, ld: int):
         ed.token_offs_pad[bm] = rest[i]
         ed.block_pid_map[bm] = rest[nb + i]
         if i < n_ord:
-            ed.gemm_order[bm] = rest[2 * nb + i][:tiles[i]]
+            ed.gemm_order[bm] = rest[2 * (nb + i)]
     return gate_scal, hist, topk_indx, gate_indx, ed
 
 
