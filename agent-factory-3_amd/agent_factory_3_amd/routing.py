@@ -18,6 +18,7 @@ All index work runs in HIP kernels on the caller's stream (no host sync).
 from __future__ import annotations
 
 import ctypes
+import functools
 from dataclasses import dataclass, field
 
 import torch
@@ -182,9 +183,16 @@ class _GateScal(torch.autograd.Function):
         return dlogits.to(ctx.dtype), None, None, None, None
 
 
+@functools.lru_cache(maxsize=8)
+def _c_ints(values: tuple):
+    """``values`` as a C array (read by the call it is passed to, never written)."""
+    return (ctypes.c_int32 * len(values))(*values)
+
+
 def _routing_plan(lg: torch.Tensor, K: int, ei: torch.Tensor | None, ld: int):
-    """Routing and its tile metadata in one call (af3_routing_plan): the outputs
-    lie in one int32 buffer.  Returns (gate_scal, hist, topk_indx,
+    """Routing and its tile metadata in one call (af3_routing_plan): the index
+    outputs lie in one int32 buffer (the histogram, which a program may keep for
+    its statistics, in its own).  Returns (gate_scal, hist, topk_indx,
     gate_indx, ExptData)."""
     T, E = lg.shape
     R = T * K
@@ -194,22 +202,23 @@ def _routing_plan(lg: torch.Tensor, K: int, ei: torch.Tensor | None, ld: int):
     tiles = [max_tiles(R, E, bm) for bm in bms]
     mt = max(tiles)
     n_ord = max(bms.index(bm) for bm in GEMM_ORDER_BMS) + 1   # orders for the leading sizes
-    sizes = [E, E + 1, R, R] + [E + 1] * nb + [mt] * nb
+    sizes = [E + 1, R, R] + [E + 1] * nb + [mt] * nb
     for n in tiles[:n_ord]:   # an order's slots past its size's most tiles are not handed out
         sizes += [n, mt - n]
     buf = torch.empty(sum(sizes), dtype=torch.int32, device=dev)
+    hist = torch.empty(E, dtype=torch.int32, device=dev)
     gate_scal = torch.empty(R, dtype=torch.bfloat16, device=dev)
     lib = _capi.load()
     topk = 1 if ei is None else 0
     ws_n = int(lib.af3_routing_plan_workspace_bytes(T, E, K, topk))
     ws = torch.empty(ws_n, dtype=torch.uint8, device=dev) if ws_n else None
-    hist, offs, topk_indx, gate_indx, *rest = buf.split(sizes)
+    offs, topk_indx, gate_indx, *rest = buf.split(sizes)
     # tensors of their own to autograd: slices share one version counter, so that an
     # in-place change of one output would count as a change of those saved for backward
-    hist, offs, topk_indx, gate_indx = hist.data, offs.data, topk_indx.data, gate_indx.data
+    offs, topk_indx, gate_indx = offs.data, topk_indx.data, gate_indx.data
     _capi.call("af3_routing_plan", lg.data_ptr(), ld, _capi.ptr(ei), topk, T, E, K, gate_scal.data_ptr(),
                hist.data_ptr(), topk_indx.data_ptr(), gate_indx.data_ptr(), offs.data_ptr(),
-               (ctypes.c_int32 * nb)(*bms), nb, n_ord, mt, rest[0].data_ptr(), rest[nb].data_ptr(),
+               _c_ints(bms), nb, n_ord, mt, rest[0].data_ptr(), rest[nb].data_ptr(),
                rest[2 * nb].data_ptr(), _capi.ptr(ws), ws_n, _capi.stream_of(dev))
     ed = ExptData(hist, offs, n_gates=R)
     for i, bm in enumerate(bms):

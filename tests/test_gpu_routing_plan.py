@@ -149,6 +149,12 @@ def test_outputs_change_in_place_on_their_own(dev, monkeypatch):
     assert torch.equal(grads[0], grads[1]) and grads[0].abs().sum() > 0
 
 
+def test_kept_histogram_keeps_nothing_else(dev):
+    """A histogram kept for statistics holds its E counts alive, not the routing's index buffer."""
+    logits = torch.randn(2000, 32, device=dev).to(torch.bfloat16)
+    assert R.routing(logits, 4)[0].expt_hist.untyped_storage().nbytes() == 4 * 32
+
+
 def test_entry_points_agree(dev):
     """af3_routing_replay / _topk / _replay_noalloc give the plan's outputs."""
     for T, E, K in ((50, 32, 4), (3000, 128, 4)):
