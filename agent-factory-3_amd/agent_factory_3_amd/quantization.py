@@ -77,8 +77,9 @@ GEMM_BLOCK_M = 128
 # gradient gains 4-6% up to 12 rows (32) and 2-6% from 22 to 32 (64); between them it
 # is within 3% of the 128-row map either way (13-18 rows on 32: 0 to -3%, where the
 # 64-row map is 2-5% behind; 19-21 on 64: 0 to -3%, on 32 -5 to -7%), while even
-# loads gain 5-11% there.  Loads on a few experts only (4 or 16 of 128) lose up to 10%
-# forward and 30% in the gradient past 10 rows; the loads are not known on the host.
+# loads gain 5-11% there.  Loads on a few experts only (4 or 16 of 128) lose up to 14%
+# forward and a third in the gradient past 10 rows; the loads are not known on the
+# host.
 GEMM_TILE = {"block_m": 256, "tile_cfg": 0, "fwd_block_m": 128, "dx_block_m": 128, "short": True}
 FWD_SHORT_ROWS = ((24, 32), (48, 64))   # (rows per expert at most, block_m)
 DX_SHORT_ROWS = ((18, 32), (32, 64))
