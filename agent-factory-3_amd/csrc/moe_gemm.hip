@@ -1944,7 +1944,7 @@ __device__ __forceinline__ void d5_tile(const Params& p, uint8_t* lds, int e, in
   // work), the other's k-loop keeps issue priority for its MFMAs and copies
   if constexpr (HALF) __builtin_amdgcn_s_setprio(2);
   issue(0);
-  issue_from(min(1, nk - 1), STAGE);
+  if (nk > 1) issue(1);
 
   // TS: the exact conversion is chosen per work item (the tiled scales carry a
   // flag per expert and n-tile: any scale byte outside [2, 252]), so the
@@ -1957,7 +1957,9 @@ __device__ __forceinline__ void d5_tile(const Params& p, uint8_t* lds, int e, in
     // The k-loop is bound by instruction issue (44% of the waves' cycles issue),
     // so nothing but the data path is in it: scale bytes take one shift (the
     // conversion ignores sign and mantissa), the ring's stage offsets are carried
-    // scalars, copies and waits are unconditional.  223 instructions per k-step
+    // scalars, copies and waits are unconditional (a loop of its own runs the last
+    // two k-steps, which copy nothing: repeating copies there and waiting for them
+    // at the end cost a launch 1-2 us, 2-7% at K <= 640).  223 instructions per k-step
     // of the tiled-scale 128 x 256 item against 306 with masks, a modulo per LDS
     // address and guarded copies; a 20b layer's two launches (16384 tokens) 3163
     // -> 3020 us.
@@ -1965,11 +1967,11 @@ __device__ __forceinline__ void d5_tile(const Params& p, uint8_t* lds, int e, in
     // k-step, skipped at kt = 0) and 0..2; iteration s runs the MFMAs of
     // sub-step s while reading and converting the fragments of s + 1
     // so: the k-step's stage (LDS byte offset), nso: the one its copies (for kt + 2) go to
-    // (uniform k-steps: the last two copy the last k-step again, into stages no
-    // wave reads again, so no copy and no wait of the loop is conditional)
-    auto kstep = [&](int kt, uint32_t so, uint32_t nso, bool first) {
+    // (copies: the loop's k-steps copy unconditionally; the last two, a loop of
+    // their own, have nothing to copy)
+    auto kstep = [&](int kt, uint32_t so, uint32_t nso, bool first, bool copies) {
       const uint8_t* stg = lds + so;
-      const int nxt_copy = min(kt + 2, nk - 1);
+      const int nxt_copy = kt + 2;
       bool odd = false;
 #pragma unroll
       for (int s = -1; s < 3; ++s) {
@@ -2081,9 +2083,10 @@ __device__ __forceinline__ void d5_tile(const Params& p, uint8_t* lds, int e, in
           }
           if constexpr (HALF) {
             const int j = o * 2 + (i == 3 ? 0 : 1);
-            if ((i == 3 || i == 10) && j < NCP) issue_one(nxt_copy, nso, j);
+            if (copies && (i == 3 || i == 10) && j < NCP) issue_one(nxt_copy, nso, j);
           } else {
-            if (i == 2 || i == 7 || i == 12) issue_one(nxt_copy, nso, o * 3 + (i == 2 ? 0 : i == 7 ? 1 : 2));
+            if (copies && (i == 2 || i == 7 || i == 12))
+              issue_one(nxt_copy, nso, o * 3 + (i == 2 ? 0 : i == 7 ? 1 : 2));
           }
           __builtin_amdgcn_sched_barrier(0);
         }
@@ -2113,22 +2116,33 @@ __device__ __forceinline__ void d5_tile(const Params& p, uint8_t* lds, int e, in
 #pragma unroll
     for (int tn = 0; tn < TN; ++tn) bf[1][tn] = zf;
     // a k-step's stage is complete once this wave's copies for it have landed
-    // (the NCP newer ones may be outstanding)
-    auto wait_stage = [&] { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NCP) : "memory"); };
-    wait_stage();
-    AF3_ASM_LDS_BARRIER();
-    kstep(0, 0u, 2u * STAGE, true);
+    // (the NCP newer ones may be outstanding, none at the last k-step)
+    auto wait_stage = [&](bool last) {
+      if (last)
+        AF3_ASM_WAIT_VM(0);
+      else
+        asm volatile("s_waitcnt vmcnt(%0)" ::"n"(NCP) : "memory");
+      AF3_ASM_LDS_BARRIER();
+    };
+    wait_stage(nk == 1);
+    kstep(0, 0u, 2u * STAGE, true, nk > 2);
     // the stage of k-step kt, and that of kt + 2 = kt - 1, carried as scalars
     uint32_t so = STAGE, nso = 0u;
-#pragma nounroll
-    for (int kt = 1; kt < nk; ++kt) {
-      wait_stage();
-      AF3_ASM_LDS_BARRIER();
-      kstep(kt, so, nso, false);
+    auto next = [&] {
       nso = so;
       so = so == 2u * STAGE ? 0u : so + STAGE;
+    };
+    int kt = 1;
+#pragma nounroll
+    for (; kt + 2 < nk; ++kt, next()) {
+      wait_stage(false);
+      kstep(kt, so, nso, false, true);
     }
-    AF3_ASM_WAIT_VM(0);  // the repeated copies, before the LDS is reused
+#pragma nounroll
+    for (; kt < nk; ++kt, next()) {
+      wait_stage(kt + 1 == nk);
+      kstep(kt, so, nso, false, false);
+    }
     // the last k-step's sub-step 3
 #pragma unroll
     for (int i = 0; i < TMW * TN; ++i) {
